@@ -69,8 +69,11 @@ enum {
 
 /* ---- numerical forms --------------------------------------------------- */
 enum {
-    /* FP64 state, FP64 arithmetic in the reference's operation order.
-     * Results are bit-for-bit independent of tiling and temporal block. */
+    /* FP64 state, FP64 arithmetic in the reference's operation order, except
+     * that Rodrigues with three levels or more applies A2 to the coherence
+     * vector plane by plane where the blob's C1, C2 are rotation planes
+     * (MBH_INFO_RODR_PLANES; the same propagator to rounding).  Results are
+     * bit-for-bit independent of tiling and temporal block. */
     MBH_FORM_FP64 = 0,
     /* FP32 state storage in HBM, FP64 arithmetic in registers.  Rodrigues
      * runs in the rotated basis (z-form, needs zform_consts); two-level
@@ -252,8 +255,10 @@ typedef struct mbh_options {
  * problem admits a specialised one (pure Maxwell with every held H cell
  * starting at zero; two-level Bloch form with a diagonal Hamiltonian, a
  * real off-diagonal dipole and lossless materials, held H starting at
- * zero).  The specialised kernels drop terms that are exact zeros,
- * so the results are the same; this flag is for verifying that. */
+ * zero; FP64 Rodrigues whose C1, C2 are rotation planes).  The first two
+ * drop terms that are exact zeros, so the results are the same; the planes
+ * give the assembled A2's results to rounding.  This flag is for verifying
+ * that. */
 #define MBH_OPT_GENERIC 1u
 
 typedef struct mbh_info {
@@ -279,6 +284,10 @@ typedef struct mbh_info {
  * Hamiltonian, a real off-diagonal dipole and lossless materials, with
  * every held H cell starting at zero, is in use */
 #define MBH_INFO_BLOCH_REAL 2u
+/* mbh_info.flags: FP64 Rodrigues (three levels and up) applies A2 plane by
+ * plane (every material's C1, C2 are rotation planes of orthonormal vector
+ * pairs, as the set-up builds them) */
+#define MBH_INFO_RODR_PLANES 4u
 
 typedef struct mbh_ctx mbh_ctx;
 

@@ -300,6 +300,104 @@ void zform_yeq(uint32_t levels, const double* zq, double* yeq)
     }
 }
 
+uint64_t rodrp_stride(uint32_t levels)
+{
+    switch (levels) {
+    case 3: return algo_rodrp<3>::STRIDE;
+    case 4: return algo_rodrp<4>::STRIDE;
+    case 5: return algo_rodrp<5>::STRIDE;
+    case 6: return algo_rodrp<6>::STRIDE;
+    default: return 0;
+    }
+}
+
+/* Rotation-plane constants (layout algo_rodrp<N>) of one material from its
+ * reference blob (MBH_RODR_STRIDE).  Returns false where some plane with a
+ * nonzero angle is not C1 = q2 q1^T - q1 q2^T, C2 = -(q1 q1^T + q2 q2^T)
+ * with orthonormal q1, q2, to PLANE_TOL per entry (the entries are at most
+ * one; a Schur basis is orthonormal to some 1e-15). */
+constexpr double PLANE_TOL = 1e-13;
+
+bool rodr_planes(uint32_t levels, const double* cq, double* o)
+{
+    const int K = (int)(levels * levels) - 1, B = K / 2;
+    std::fill(o, o + rodrp_stride(levels), 0.0);
+    if (cq[0] == 0.0) {
+        return true;
+    }
+    const double* M = cq + 5;
+    const double* A1 = M + 3 * K * K;
+    const double* v = A1 + K * K;
+    const double* d_eq = v + K;
+    const double* d_in = d_eq + K;
+    const double* th = d_in + K;
+    const double* C1 = th + B;
+    const double* C2 = C1 + (size_t)B * K * K;
+    double* c = o + 4;
+    double* pv = c + K;
+    double* pl = pv + K + K * K;
+    o[0] = 1.0;
+    long double pb = 0.0L;
+    for (int i = 0; i < K; i++) {
+        const long double w = (long double)cq[1] * v[i];
+        long double acc = -(long double)d_in[i], col = 0.0L;
+        for (int k = 0; k < K; k++) {
+            acc += (long double)A1[i * K + k] * d_in[k];
+            col += (long double)cq[1] * v[k] * M[k * K + i];
+        }
+        c[i] = (double)acc;
+        pv[i] = (double)col;
+        pb += w * d_eq[i];
+    }
+    o[2] = (double)pb;
+    std::copy(A1, A1 + K * K, pv + K);
+    int np = 0;
+    for (int b = 0; b < B; b++) {
+        if (th[b] == 0.0) {
+            continue; /* sin = 1 - cos = 0 */
+        }
+        const double* P1 = C1 + (size_t)b * K * K;
+        const double* P2 = C2 + (size_t)b * K * K;
+        int m = 0;
+        for (int k = 1; k < K; k++) {
+            m = (-P2[k * K + k] > -P2[m * K + m]) ? k : m;
+        }
+        if (!(-P2[m * K + m] > 0.0)) {
+            return false;
+        }
+        double* q1 = pl + 1;
+        double* q2 = pl + 1 + K;
+        const double nrm = std::sqrt(-P2[m * K + m]);
+        for (int k = 0; k < K; k++) {
+            q1[k] = -P2[k * K + m] / nrm;
+        }
+        for (int i = 0; i < K; i++) {
+            long double acc = 0.0L;
+            for (int k = 0; k < K; k++) {
+                acc += (long double)P1[i * K + k] * q1[k];
+            }
+            q2[i] = (double)acc;
+        }
+        for (int i = 0; i < K; i++) {
+            for (int k = 0; k < K; k++) {
+                const double e1 = q2[i] * q1[k] - q1[i] * q2[k];
+                const double e2 = -(q1[i] * q1[k] + q2[i] * q2[k]);
+                /* (negated, so that a NaN fails) */
+                if (!(std::fabs(P1[i * K + k] - e1) <= PLANE_TOL &&
+                      std::fabs(P2[i * K + k] - e2) <= PLANE_TOL)) {
+                    return false;
+                }
+            }
+        }
+        pl[0] = th[b] * cq[2];
+        o[3] = std::max(o[3], std::fabs(pl[0]));
+        pl += 1 + 2 * K;
+        np++;
+    }
+    o[1] = (double)np;
+    return true;
+}
+
 /* MFMA-form constants of one material (layout zm_geom<N>) from its
  * z-form blob (layout algo_zform<N>): split FP16 fragments of the scaled
  * W - I in the kernel's row order, and per-lane rows of theta, a, c and
@@ -445,6 +543,7 @@ struct mbh_ctx {
      * applies) */
     bool bloch_real = false;
     bool generic = false; /* MBH_OPT_GENERIC: no specialised kernels */
+    bool planes = false;  /* FP64 Rodrigues by rotation planes (algo_rodrp) */
     std::vector<int32_t> mat_h; /* per super-grid cell (Bloch conversions) */
     std::vector<double> qm_h;   /* device blob copy (Bloch conversions) */
 
@@ -939,6 +1038,9 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
     if (ctx->bloch && ctx->bloch_real && ctx->hz_zero && !ctx->generic) {
         kform = ctx->fp32 ? KFORM_BLOCH2R_MIXED : KFORM_BLOCH2R_ZFORM64;
     }
+    if (ctx->planes) {
+        kform = KFORM_RODR_PLANES;
+    }
     ctx->kform = kform;
     std::vector<uint32_t> cs;
     /* cells per lane (tiles of several wavefronts count as their cells
@@ -1276,6 +1378,25 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
     }
     c->generic = (opt.flags & MBH_OPT_GENERIC) != 0;
     const size_t esz = c->fp32 ? sizeof(float) : sizeof(double);
+    /* FP64 Rodrigues, three levels and up: by rotation planes where every
+     * material's C1, C2 have that form (what the set-up builds); 4 K FMAs
+     * per plane instead of 4 K^2 operations */
+    std::vector<double> planes;
+    if (c->algo == MBH_ALGO_CVR_RODR && c->levels >= 3 &&
+        c->form == MBH_FORM_FP64 && !c->generic) {
+        const uint64_t ps = rodrp_stride(c->levels);
+        c->planes = true;
+        for (uint32_t r = 0; r < num_runs && c->planes; r++) {
+            for (uint32_t m = 0; m < runs[r].num_materials && c->planes;
+                 m++) {
+                planes.resize(planes.size() + ps);
+                c->planes = rodr_planes(
+                    c->levels,
+                    runs[r].qm_consts + (size_t)m * runs[r].qm_stride,
+                    &planes[planes.size() - ps]);
+            }
+        }
+    }
 
     /* super-grid layout */
     uint64_t G = 0, scratch_total = 0;
@@ -1304,6 +1425,9 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
         c->zform ? runs[0].zform_stride : runs[0].qm_stride;
     c->qstride = c->bloch ? BLOCH2_STRIDE
                           : (c->zform ? src_stride + c->dref : src_stride);
+    if (c->planes) {
+        c->qstride = rodrp_stride(c->levels);
+    }
     std::vector<double> qm((size_t)nmat_total * c->qstride);
     uint32_t moff = 0;
     for (uint32_t r = 0; r < num_runs; r++) {
@@ -1323,6 +1447,10 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
             if (c->bloch) {
                 bloch2_constants(q + (size_t)m * p.qm_stride,
                                  &qm[(size_t)(moff + m) * c->qstride]);
+            } else if (c->planes) {
+                std::copy_n(&planes[(size_t)(moff + m) * c->qstride],
+                            c->qstride,
+                            &qm[(size_t)(moff + m) * c->qstride]);
             } else if (c->qstride) {
                 double* dst = &qm[(size_t)(moff + m) * c->qstride];
                 std::memcpy(dst, q + (size_t)m * src_stride,
@@ -1961,6 +2089,9 @@ int mbh_get_info(const mbh_ctx* ctx, mbh_info* info)
     if (ctx->kform == KFORM_BLOCH2R_MIXED ||
         ctx->kform == KFORM_BLOCH2R_ZFORM64) {
         info->flags |= MBH_INFO_BLOCH_REAL;
+    }
+    if (ctx->kform == KFORM_RODR_PLANES) {
+        info->flags |= MBH_INFO_RODR_PLANES;
     }
     return MBH_OK;
 }

@@ -772,6 +772,271 @@ __device__ __forceinline__ void tier_sincos(double x, double& s, double& c)
 }
 
 /* ======================================================================
+ * lindblad_cvr_rodr<N>::update with A2 applied to the vector instead of
+ * assembled.  Each rotation plane b of the dipole Liouvillian is spanned by
+ * two orthonormal vectors q1, q2 with C1_b = q2 q1^T - q1 q2^T and
+ * C2_b = -(q1 q1^T + q2 q2^T), so with alpha = q1.d, beta = q2.d
+ *   A2 d = d + sum_b q1 (-sin beta - (1 - cos) alpha)
+ *                  + q2 ( sin alpha - (1 - cos) beta):
+ * 4 K FMAs per plane where building A2 takes 4 K^2 operations per plane.
+ * The host recovers the vectors from the blob's C1 and C2 and checks that
+ * they reproduce both; a blob that is not of this form (and
+ * MBH_OPT_GENERIC) takes algo_rodr, which accepts any C1, C2.
+ * The half steps are A1 d + c with c = (A1 - I) d_in, and
+ * p = pv.d + pb with pv = M_CP v^T M, pb = M_CP v.d_eq.  The basis stays
+ * that of the coherence vector, so exact zeros of A1, pv and the planes
+ * stay exact (a run that starts from noise has p = 0 until its coherences
+ * grow, as in the reference form).  State: d, as algo_rodr.
+ * Bound by the latency of one step's chain on grids that leave the SIMDs
+ * one wavefront or none.  Whole runs, algo_rodr -> algo_rodrp: six-level
+ * ladder, 8192 cells x 800 steps, 1702 -> 18.6 ms (algo_rodr: 93 kflop and
+ * 10 KB of scratch per lane and step); five-level comb, 8192 x 600,
+ * 239 -> 5.3 ms; three levels, 16384 x 8000, 112 -> 16.7 ms, and one cell,
+ * 10000 steps, 102 -> 34 ms.
+ *
+ * Blob (STRIDE doubles): [0] has_qm  [1] number of planes  [2] pb
+ *   [3] max theta dt   then c (K), pv (K), A1 (K^2),
+ *   planes: B x { theta dt, q1 (K), q2 (K) }
+ * ==================================================================== */
+/* sin(x) and 1 - cos(x) of one cell's plane angles, by the cell's own range
+ * (the results of a cell do not depend on its neighbours): SMALL |x| <=
+ * 2^-5, Taylor to x^9 and x^8 (relative truncation below 1e-18); MEDIUM
+ * |x| <= 0.25 (to x^13 / x^14); else the library. */
+constexpr double PLANE_SMALL = 0.03125;
+
+__device__ __forceinline__ void plane_sincos(double x, bool small, bool medium,
+                                             bool all_small, bool all_medium,
+                                             double& s, double& v)
+{
+    const double x2 = x * x;
+    double ps = 2.7557319223985890653e-06;        /* 1/9! */
+    ps = fma(ps, x2, -1.9841269841269841270e-04); /* -1/7! */
+    ps = fma(ps, x2, 8.3333333333333333333e-03);  /* 1/5! */
+    ps = fma(ps, x2, -1.6666666666666666667e-01); /* -1/3! */
+    s = fma(ps * x2, x, x);
+    double pc = -2.4801587301587301587e-05;       /* -1/8! */
+    pc = fma(pc, x2, 1.3888888888888888889e-03);  /* 1/6! */
+    pc = fma(pc, x2, -4.1666666666666666667e-02); /* -1/4! */
+    pc = fma(pc, x2, 0.5);                        /* 1/2! */
+    v = pc * x2;
+    if (!all_small) {
+        double qs = 1.6059043836821614599e-10;        /* 1/13! */
+        qs = fma(qs, x2, -2.5052108385441718775e-08); /* -1/11! */
+        qs = fma(qs, x2, 2.7557319223985890653e-06);
+        qs = fma(qs, x2, -1.9841269841269841270e-04);
+        qs = fma(qs, x2, 8.3333333333333333333e-03);
+        qs = fma(qs, x2, -1.6666666666666666667e-01);
+        double s2 = fma(qs * x2, x, x);
+        double qc = 1.1470745597729724714e-11;        /* 1/14! */
+        qc = fma(qc, x2, -2.0876756987868098979e-09); /* -1/12! */
+        qc = fma(qc, x2, 2.7557319223985890653e-07);  /* 1/10! */
+        qc = fma(qc, x2, -2.4801587301587301587e-05);
+        qc = fma(qc, x2, 1.3888888888888888889e-03);
+        qc = fma(qc, x2, -4.1666666666666666667e-02);
+        qc = fma(qc, x2, 0.5);
+        double v2 = qc * x2;
+        if (!all_medium) {
+            double sl, cl;
+            sincos(x, &sl, &cl);
+            s2 = medium ? s2 : sl;
+            v2 = medium ? v2 : 1.0 - cl;
+        }
+        s = small ? s : s2;
+        v = small ? v : v2;
+    }
+}
+
+template<int N>
+struct algo_rodrp {
+    static constexpr bool SHIFT = false;
+    static constexpr bool FAST_FDTD = false;
+    static constexpr int K = N * N - 1;
+    static constexpr int B = K / 2;
+    static constexpr int DC = K;
+    static constexpr int STATE = K;
+    struct state {
+        double v[STATE];
+    };
+
+    static constexpr int OFF_C = 4;
+    static constexpr int OFF_PV = OFF_C + K;
+    static constexpr int OFF_A1 = OFF_PV + K;
+    static constexpr int OFF_PL = OFF_A1 + K * K;
+    static constexpr int PLANE = 1 + 2 * K;
+    static constexpr int STRIDE = OFF_PL + B * PLANE;
+
+    /* three levels: the 155 constants are staged in LDS (they do not fit
+     * the SGPRs), as for the z-form */
+    static constexpr int STAGE = (K <= 8) ? STRIDE : 0;
+
+    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
+
+    /* o = A1 d + c: every row accumulates in ascending order; RG rows side
+     * by side hide the FMA latency (more would spill at K = 35) */
+    template<int C, typename P>
+    __device__ static void half_step(P q, const double (*d)[K],
+                                     double (*o)[K])
+    {
+        const P c0 = q + OFF_C;
+        const P A1 = q + OFF_A1;
+        constexpr int RG = C != 1 ? 1 : (K <= 8 ? K : (K <= 24 ? 4 : 2));
+#pragma unroll
+        for (int i0 = 0; i0 < K; i0 += RG) {
+            double acc[C][RG];
+#pragma unroll
+            for (int g = 0; g < RG; g++) {
+                if (i0 + g < K) {
+                    const double ci = c0[i0 + g];
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        acc[c][g] = ci;
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+#pragma unroll
+                for (int g = 0; g < RG; g++) {
+                    if (i0 + g < K) {
+                        const double a = A1[(i0 + g) * K + k];
+#pragma unroll
+                        for (int c = 0; c < C; c++) {
+                            acc[c][g] = fma(a, d[c][k], acc[c][g]);
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < RG; g++) {
+                if (i0 + g < K) {
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        o[c][i0 + g] = acc[c][g];
+                    }
+                }
+            }
+        }
+    }
+
+    template<int C, typename P>
+    __device__ static void update_multi_p(P q, state* s, const double* e,
+                                          double* p)
+    {
+        double d[C][K], r[C][K];
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                r[c][k] = s[c].v[k];
+            }
+        }
+        bool small[C], medium[C];
+        bool all_s = true, all_m = true;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const double xm = q[3] * fabs(e[c]);
+            small[c] = xm <= PLANE_SMALL;
+            medium[c] = xm <= TAYLOR_MAX;
+            all_s = all_s && small[c];
+            all_m = all_m && medium[c];
+        }
+        all_s = __all(all_s);
+        all_m = __all(all_m);
+        const int np = (int)q[1];
+        /* one copy of the half step in a loop of two; the offset that the
+         * compiler cannot see through keeps A1's loads inside (kept for
+         * the second half, A1 would spill) */
+#pragma unroll 1
+        for (int half = 0;; half++) {
+            int off = 0;
+            asm volatile("" : "+s"(off));
+            half_step<C>(q + off, r, d);
+            if (half == 1) {
+                break;
+            }
+            /* the planes: r = A2 d */
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    r[c][k] = d[c][k];
+                }
+            }
+            P pl = q + off + OFF_PL;
+#pragma unroll 1
+            for (int b = 0; b < np; b++, pl += PLANE) {
+                const P q1 = pl + 1;
+                const P q2 = pl + 1 + K;
+                double u1[C], u2[C];
+#pragma unroll
+                for (int c = 0; c < C; c++) {
+                    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+#pragma unroll
+                    for (int k = 0; k < K; k++) {
+                        if (k & 1) {
+                            a1 = fma(q1[k], d[c][k], a1);
+                            b1 = fma(q2[k], d[c][k], b1);
+                        } else {
+                            a0 = fma(q1[k], d[c][k], a0);
+                            b0 = fma(q2[k], d[c][k], b0);
+                        }
+                    }
+                    const double al = a0 + a1, be = b0 + b1;
+                    double sn, vc;
+                    plane_sincos(pl[0] * e[c], small[c], medium[c], all_s,
+                                 all_m, sn, vc);
+                    u1[c] = fma(-sn, be, -(vc * al));
+                    u2[c] = fma(sn, al, -(vc * be));
+                }
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        r[c][k] =
+                            fma(q1[k], u1[c], fma(q2[k], u2[c], r[c][k]));
+                    }
+                }
+            }
+        }
+        const P pv = q + OFF_PV;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            double p0 = q[2], p1 = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                s[c].v[k] = d[c][k];
+                if (k & 1) {
+                    p1 = fma(pv[k], d[c][k], p1);
+                } else {
+                    p0 = fma(pv[k], d[c][k], p0);
+                }
+            }
+            p[c] = p0 + p1;
+        }
+    }
+
+    template<int C>
+    __device__ static void update_multi(cdp q, state* s, const double* e,
+                                        double* p)
+    {
+        update_multi_p<C>(q, s, e, p);
+    }
+    __device__ static void update(cdp q, state& s, double e, double& p)
+    {
+        update_multi<1>(q, &s, &e, &p);
+    }
+
+    __device__ static double inversion(cdp, const state& s)
+    {
+        return s.v[N * (N - 1)];
+    }
+    __device__ static double population(cdp, const state& s, int m)
+    {
+        return cv_population<N>(s.v, m);
+    }
+};
+
+/* ======================================================================
  * Rodrigues in the rotated basis (z-form).  Mathematically identical to
  * algo_rodr (A2(e) = Q R(e) Q^T, Strang halves merged into W); see the
  * zform blob description in mbsolve_hip.h.  State: y (K values).

@@ -12,6 +12,11 @@ namespace mbh {
     kernel_entry { ALGO_ID, LEV, MBH_FORM_FP64, C,                            \
                    &launch_tile<A, C, double, true>, MBH_ORDER_RED }
 
+#define MBH_RED_PLANES(LEV, C)                                                \
+    kernel_entry { MBH_ALGO_CVR_RODR, LEV, KFORM_RODR_PLANES, C,              \
+                   &launch_tile<algo_rodrp<LEV>, C, double, true>,            \
+                   MBH_ORDER_RED }
+
 template __global__ void tile_kernel<algo_noop, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_noop, 2, double, true>(KArgs);
 template __global__ void tile_kernel<algo_noop, 4, double, true>(KArgs);
@@ -28,6 +33,11 @@ template __global__ void tile_kernel<algo_rodr<3>, 2, double, true>(KArgs);
 template __global__ void tile_kernel<algo_rodr<4>, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_rodr<5>, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_rodr<6>, 1, double, true>(KArgs);
+template __global__ void tile_kernel<algo_rodrp<3>, 1, double, true>(KArgs);
+template __global__ void tile_kernel<algo_rodrp<3>, 2, double, true>(KArgs);
+template __global__ void tile_kernel<algo_rodrp<4>, 1, double, true>(KArgs);
+template __global__ void tile_kernel<algo_rodrp<5>, 1, double, true>(KArgs);
+template __global__ void tile_kernel<algo_rodrp<6>, 1, double, true>(KArgs);
 
 #if !defined(__HIP_DEVICE_COMPILE__)
 const kernel_entry k_table_red[] = {
@@ -47,6 +57,8 @@ const kernel_entry k_table_red[] = {
     MBH_RED_ENTRY(MBH_ALGO_CVR_RODR, 4, 1, algo_rodr<4>),
     MBH_RED_ENTRY(MBH_ALGO_CVR_RODR, 5, 1, algo_rodr<5>),
     MBH_RED_ENTRY(MBH_ALGO_CVR_RODR, 6, 1, algo_rodr<6>),
+    MBH_RED_PLANES(3, 1), MBH_RED_PLANES(3, 2), MBH_RED_PLANES(4, 1),
+    MBH_RED_PLANES(5, 1), MBH_RED_PLANES(6, 1),
 };
 const uint32_t k_table_red_n = sizeof(k_table_red) / sizeof(k_table_red[0]);
 #endif

@@ -100,6 +100,8 @@ constexpr int32_t TILE_MAT_QM = 0x40000000;
 constexpr uint32_t KFORM_NOOP_HZ0 = 0x100;
 constexpr uint32_t KFORM_BLOCH2R_MIXED = 0x101;
 constexpr uint32_t KFORM_BLOCH2R_ZFORM64 = 0x102;
+/* algo_rodrp (FP64 Rodrigues by rotation planes), both step orders */
+constexpr uint32_t KFORM_RODR_PLANES = 0x103;
 
 template<typename ST>
 __device__ __forceinline__ double ld(const void* p, uint64_t i)

@@ -524,3 +524,82 @@ def test_multi_wavefront_tiles_in_a_batch(gpu, tile):
         for a, c in zip(out[0][r], out[1][r]):
             assert np.max(np.abs(a)) > 0
             assert np.array_equal(a, c), (tile, r)
+
+
+def _fp64_close(prob, got, want):
+    """Populations and the inversion on the trace-1 scale, fields and p
+    relative to their maximum, each to the FP64 form's 1e-12 (a few hundred
+    steps of some tens of roundings each)."""
+    for r, a, b in zip(prob["records"], capi.split_records(prob, got),
+                       capi.split_records(prob, want)):
+        assert np.max(np.abs(b)) > 0.0, r["type"]
+        err = (float(np.max(np.abs(a - b)))
+               if r["type"] >= 3  # density, inversion
+               else rel_err(a, b))
+        assert err <= 1e-12, (r["type"], err)
+
+
+def _planes_spec(levels):
+    """Ladder of `levels` levels between vacuum margins: the field at the
+    source passes through all three ranges of the plane angle (up to about
+    1.3 rad per step at the peak), records of every kind."""
+    spec = setups.marskar2011(levels, num_gridpoints=300, endtime=0.02e-12)
+    spec["regions"] = [("v0", "Vacuum", 0.0, 3e-5),
+                       ("Active region", "AR_Marsk", 3e-5, 7e-5),
+                       ("v1", "Vacuum", 7e-5, 1e-4)]
+    spec["endtime"] = 0.3e-12
+    spec["sources"][0].update(tau=20e-15, phase=60e-15, ampl=6e9)
+    iv = spec["endtime"] / 12
+    spec["records"] = [{"name": n, "interval": iv} for n in
+                       ("inv12", "e", "h", "p")]
+    spec["records"] += [{"name": "d%d%d" % (i, i), "type": 3, "row": i,
+                         "col": i, "interval": 0.0, "position": 4e-5}
+                        for i in range(1, levels + 1)]
+    return spec
+
+
+@pytest.mark.parametrize("order", ["plain", "red"])
+@pytest.mark.parametrize("levels", [3, 4, 5, 6])
+def test_rodrigues_planes(gpu, levels, order):
+    """FP64 Rodrigues by rotation planes: the oracle's records to the FP64
+    form's bound, the same bits for every tiling, and the assembled-A2
+    kernel for blobs that are not rotation planes (one C1 entry changed by
+    1e-6) and with MBH_OPT_GENERIC."""
+    spec = _planes_spec(levels)
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, "", order), dev, scen)
+    nt = int(prob["num_timesteps"])
+    ref = oracle.OracleRun(prob).run(order=order)
+    base = None
+    tiles = (64, 128) if levels == 3 else (64,)
+    for tb, tile in [(1, 64), (7, 64)] + [(16, t) for t in tiles]:
+        print("case planes", levels, order, tb, tile, flush=True)
+        ctx = capi.Context([prob], capi.options(
+            "fp64", temporal_block=tb, tile_cells=tile, order=order))
+        assert ctx.info()["flags"] & capi.MBH_INFO_RODR_PLANES
+        ctx.run(0, nt)
+        got, st = ctx.records(0), ctx.state(0)
+        ctx.close()
+        if base is None:
+            base = (got, st)
+            _fp64_close(prob, got, ref.scratch)
+        assert np.array_equal(got, base[0])
+        for k in ("e", "h", "p", "d"):
+            assert np.array_equal(st[k], base[1][k]), k
+    K, B = levels * levels - 1, (levels * levels - 1) // 2
+    other = dict(prob)
+    q = np.array(prob["qm_consts"], dtype=float)
+    has = [m for m in range(int(prob["num_materials"]))
+           if q[m * int(prob["qm_stride"])] != 0.0][0]
+    q[has * int(prob["qm_stride"]) + 5 + 4 * K * K + 3 * K + B + 1] += 1e-6
+    other["qm_consts"] = q
+    for p, generic in ((other, False), (prob, True)):
+        print("case general", levels, order, generic, flush=True)
+        ctx = capi.Context([p], capi.options("fp64", temporal_block=8,
+                                             order=order, generic=generic))
+        assert not ctx.info()["flags"] & capi.MBH_INFO_RODR_PLANES
+        ctx.run(0, 300)
+        got = ctx.records(0)
+        ctx.close()
+        _fp64_close(p, got, oracle.OracleRun(p).run(0, 300,
+                                                    order=order).scratch)
