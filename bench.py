@@ -81,7 +81,7 @@ STORAGE = {"mixed": "f32", "mfma": "f32", "zform": "f64", "mfma64": "f64",
 EXACT64 = ("zform", "")
 # v_mfma_f32_16x16x32_f16 per 16-cell block and step (split products x
 # M-tiles x K chunks)
-MFMA_PER_BLOCK = {6: 18, 5: 6, 4: 3, 3: 4}
+MFMA_PER_BLOCK = {6: 18, 5: 6, 4: 3}
 MFMA_FLOPS = 2 * 16 * 16 * 32
 LEVELS = {"qcl6": 6, "sweep6": 6, "v3": 3, "sit2": 2, "sweep2": 2,
           "maxwell": 0}
@@ -575,7 +575,7 @@ def main():
     units_per_launch = cu_pass / max(launches, 1)
     achieved = bpu * units_per_launch / (launch_ms * 1e-3) / 1e9
     lev = LEVELS[args.config]
-    mfma_form = head.startswith("mfma")
+    mfma_form = head.startswith("mfma") and info["mfma_tiles"] > 0
     out = {
         "metric": "cell-updates/s, mixed vs FP64 GPU at <=1e-5 rel err; "
                   "% HBM/MFMA roofline",

@@ -87,9 +87,11 @@ enum {
     MBH_FORM_ZFORM64 = 2,
     /* Rodrigues z-form, N = 3..6, FP32 state storage: rotation, affine part
      * and p in FP64, the generator product (W - I) r on the matrix cores as
-     * FP16 hi + lo split products with FP32 accumulation. */
+     * FP16 hi + lo split products with FP32 accumulation for four levels and
+     * up; for three levels, where that is slower, in FP64 as MBH_FORM_MIXED. */
     MBH_FORM_MFMA = 3,
-    /* as MBH_FORM_MFMA with FP64 state storage */
+    /* as MBH_FORM_MFMA with FP64 state storage (three levels: as
+     * MBH_FORM_ZFORM64) */
     MBH_FORM_MFMA64 = 4
 };
 

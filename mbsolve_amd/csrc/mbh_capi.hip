@@ -89,7 +89,7 @@ __global__ void bloch_to_ref(const ST* __restrict__ sig, uint64_t dstride,
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
          i < cells; i += stride) {
         const uint64_t g = base + i;
-        const double* o = qm + (uint64_t)mat[g] * qstride;
+        const double* o = qm + (uint64_t)mat_of(mat[g]) * qstride;
         double sv[4], rho[4];
         for (int j = 0; j < 4; j++) {
             sv[j] = (double)sig[(uint64_t)j * dstride + g];
@@ -146,6 +146,8 @@ constexpr uint32_t BLOCH_FROM_REF[4] = { 0, 6, 2, 3 };
 
 /* Bloch-form constants (layout in algo_bloch2) from the reference Cayley
  * blob of a two-level material (MBH_CAYLEY_STRIDE(2) doubles). */
+constexpr double TRACE_TOL = 2e-15;
+
 void bloch2_constants(const double* cq, double* o)
 {
     typedef std::complex<double> cx;
@@ -246,6 +248,15 @@ void bloch2_constants(const double* cq, double* o)
     }
     o[26] = g;
     o[27] = std::fma(o[7], o[7], 1.0); /* 1 + alpha0^2 at e = 0 */
+    o[28] = o[3] * o[3];
+    /* scattering keeps the trace, F = (1, 0; ...) exactly; the rounding of
+     * D1 and of the products above leaves it off by a few 1e-16 per step,
+     * which would add up over a run */
+    if (std::fabs(o[10] - 1.0) <= TRACE_TOL &&
+        std::fabs(o[11]) <= TRACE_TOL) {
+        o[10] = 1.0;
+        o[11] = 0.0;
+    }
 }
 
 /* reference (rho00, rho11, Re rho01, Im rho01) -> carried Bloch state
@@ -297,6 +308,44 @@ void zform_yeq(uint32_t levels, const double* zq, double* yeq)
             acc += Qt[i * K + j] * din[j];
         }
         yeq[i] = (zq[0] != 0.0) ? -acc : 0.0;
+    }
+}
+
+uint64_t zform_stride_dev(uint32_t levels)
+{
+    switch (levels) {
+    case 2: return algo_zform<2>::DEV_STRIDE;
+    case 3: return algo_zform<3>::DEV_STRIDE;
+    case 4: return algo_zform<4>::DEV_STRIDE;
+    case 5: return algo_zform<5>::DEV_STRIDE;
+    case 6: return algo_zform<6>::DEV_STRIDE;
+    default: return 0;
+    }
+}
+
+/* Populations of a z-form blob as linear forms of y (OFF_POP): with
+ * d = P y + o and rho_mm = 1 / N + sum_i f_i d_(N(N-1)+i) / 2,
+ * f_i = -1, m or 0 (m < i + 1, m = i + 1, m > i + 1) over
+ * sqrt((i + 1)(i + 2) / 2) (cv_population). */
+void zform_pop(uint32_t levels, const double* zq, double* out)
+{
+    const int N = (int)levels, K = N * N - 1, B = K / 2;
+    const double* P = zq + 3 + B + K * K + 2 * K;
+    const double* o = P + K * K;
+    for (int m = 0; m < N; m++) {
+        double* r = out + (size_t)m * (K + 1);
+        for (int j = 0; j <= K; j++) {
+            long double acc = j == K ? 1.0L / N : 0.0L;
+            for (int i = 0; zq[0] != 0.0 && i < N - 1; i++) {
+                const long double f = m < i + 1 ? -1.0L
+                                                : (m == i + 1 ? m : 0.0L);
+                const int row = N * (N - 1) + i;
+                acc += 0.5L * f /
+                    std::sqrt((long double)(((i + 1) * (i + 2)) / 2)) *
+                    (j == K ? o[row] : P[(size_t)row * K + j]);
+            }
+            r[j] = (double)acc;
+        }
     }
 }
 
@@ -454,17 +503,10 @@ void zm_build(const double* zq, unsigned char* out)
                         v = cv[i] * sc;
                     }
                     const _Float16 hi = (_Float16)v;
-                    const double r1 = v - (double)hi;
-                    const _Float16 mid = (_Float16)r1;
-                    const _Float16 lo = (_Float16)(r1 - (double)mid);
                     const int f = (t * Gm::KC + kc) * Gm::AP;
                     fr[(f * 64 + l) * 8 + sl] = hi;
-                    if (Gm::AP == 3) {
-                        fr[((f + 1) * 64 + l) * 8 + sl] = mid;
-                        fr[((f + 2) * 64 + l) * 8 + sl] = lo;
-                    } else {
-                        fr[((f + 1) * 64 + l) * 8 + sl] = (_Float16)r1;
-                    }
+                    fr[((f + 1) * 64 + l) * 8 + sl] =
+                        (_Float16)(v - (double)hi);
                 }
             }
         }
@@ -502,7 +544,6 @@ void zm_build(const double* zq, unsigned char* out)
 uint64_t zm_bytes(uint32_t levels)
 {
     switch (levels) {
-    case 3: return zm_geom<3>::BYTES;
     case 4: return zm_geom<4>::BYTES;
     case 5: return zm_geom<5>::BYTES;
     case 6: return zm_geom<6>::BYTES;
@@ -513,7 +554,6 @@ uint64_t zm_bytes(uint32_t levels)
 void zm_build_levels(uint32_t levels, const double* zq, unsigned char* out)
 {
     switch (levels) {
-    case 3: zm_build<3>(zq, out); break;
     case 4: zm_build<4>(zq, out); break;
     case 5: zm_build<5>(zq, out); break;
     case 6: zm_build<6>(zq, out); break;
@@ -581,10 +621,8 @@ struct mbh_ctx {
     uint64_t n_tiles_mfma = 0;      /* uniform tiles of a density material */
     std::vector<uint8_t> mat_has_qm; /* per material (MFMA forms) */
     dev_source* src = nullptr;
-    uint32_t* tile_src = nullptr;
-    dev_record* rec = nullptr;
-    uint32_t* tile_rec_ptr = nullptr;
-    uint32_t* tile_rec_idx = nullptr;
+    tile_meta* tiles = nullptr;
+    dev_record* tile_rec = nullptr;
     double* src_data = nullptr;
     double* rec_buf = nullptr; /* record scratch of all runs */
     uint64_t rec_total = 0;    /* doubles in rec_buf */
@@ -872,11 +910,27 @@ const kernel_entry* find_kernel(uint32_t algo, uint32_t levels, uint32_t form,
     return nullptr;
 }
 
+/* The MFMA kernel is for four levels and up: on three the VALU z-form is
+ * faster (the 8 x 8 product fills a quarter of an MFMA's output tile) and
+ * exact to FP64, so the MFMA forms run it with their own state storage. */
+bool on_matrix_cores(uint32_t levels, uint32_t form)
+{
+    return levels >= 4 && (form == MBH_FORM_MFMA || form == MBH_FORM_MFMA64);
+}
+
 /* Kernel form implementing the requested numerical form: Rodrigues and
  * two-level Cayley have restructured kernels for MIXED and ZFORM64; the
  * others fall back to the reference operation order (ZFORM64 -> FP64). */
 uint32_t kernel_form(uint32_t algo, uint32_t levels, uint32_t form)
 {
+    if (algo == MBH_ALGO_CVR_RODR && levels == 3) {
+        if (form == MBH_FORM_MFMA) {
+            return MBH_FORM_MIXED;
+        }
+        if (form == MBH_FORM_MFMA64) {
+            return MBH_FORM_ZFORM64;
+        }
+    }
     const bool restructured = (algo == MBH_ALGO_CVR_RODR) ||
         (algo == MBH_ALGO_REG_CAYLEY && levels == 2);
     if (!restructured && form == MBH_FORM_ZFORM64) {
@@ -910,7 +964,7 @@ void set_geometry(mbh_ctx* ctx, uint32_t C, uint32_t tb)
 int build_tile_tables(mbh_ctx* ctx, bool with_records)
 {
     const uint64_t nt = ctx->num_tiles;
-    std::vector<uint32_t> ts(2 * nt);
+    std::vector<tile_meta> meta(nt, tile_meta{ 0, 0, 0, 0 });
     for (uint64_t t = 0; t < nt; t++) {
         const int64_t lo = (int64_t)(t * ctx->owned) - ctx->halo;
         const int64_t hi = lo + 64 * (int64_t)ctx->C;
@@ -922,10 +976,10 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
                                   [](const dev_source& s, int64_t v) {
                                       return (int64_t)s.gx < v;
                                   });
-        ts[2 * t] = (uint32_t)(a - ctx->srcs.begin());
-        ts[2 * t + 1] = (uint32_t)(b - ctx->srcs.begin());
+        meta[t].src_lo = (uint32_t)(a - ctx->srcs.begin());
+        meta[t].src_hi = (uint32_t)(b - ctx->srcs.begin());
     }
-    std::vector<uint32_t> ptr(nt + 1, 0), idx;
+    std::vector<dev_record> recs;
     if (with_records) {
         std::vector<std::pair<uint64_t, uint32_t>> tile_rec;
         for (uint32_t id = 0; id < ctx->recs.size(); id++) {
@@ -941,13 +995,19 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
                             const std::pair<uint64_t, uint32_t>& y) {
                              return x.first < y.first;
                          });
-        idx.reserve(tile_rec.size());
+        recs.reserve(tile_rec.size());
+        uint64_t t = 0;
         for (auto& tr : tile_rec) {
-            ptr[tr.first + 1]++;
-            idx.push_back(tr.second);
+            for (; t < tr.first; t++) {
+                meta[t].rec_hi = meta[t + 1].rec_lo = (uint32_t)recs.size();
+            }
+            recs.push_back(ctx->recs[tr.second]);
         }
-        for (uint64_t t = 0; t < nt; t++) {
-            ptr[t + 1] += ptr[t];
+        for (; t < nt; t++) {
+            meta[t].rec_hi = (uint32_t)recs.size();
+            if (t + 1 < nt) {
+                meta[t + 1].rec_lo = (uint32_t)recs.size();
+            }
         }
     }
     /* replace the previous tables */
@@ -961,12 +1021,12 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
         }
         (void)hipFree(p);
     };
-    release(ctx->tile_src);
-    release(ctx->tile_rec_ptr);
-    release(ctx->tile_rec_idx);
+    release(ctx->tiles);
+    release(ctx->tile_rec);
     release(ctx->tiles_a);
     release(ctx->tiles_mat);
-    ctx->tile_src = ctx->tile_rec_ptr = ctx->tile_rec_idx = nullptr;
+    ctx->tiles = nullptr;
+    ctx->tile_rec = nullptr;
     ctx->tiles_a = nullptr;
     ctx->tiles_mat = nullptr;
     ctx->n_tiles_mixed = 0;
@@ -997,7 +1057,7 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
         for (size_t i = ctx->n_tiles_mixed; i < lb.size(); i++) {
             const int64_t lo = (int64_t)(lb[i] * ctx->owned) - ctx->halo;
             const int32_t m0 = ctx->mat_h[lo];
-            lm[i] = m0 | (ctx->mat_has_qm[(size_t)m0] ? TILE_MAT_QM : 0);
+            lm[i] = m0 | (ctx->mat_has_qm[(size_t)m0] ? MAT_QM : 0);
         }
         if ((rc = upload(ctx, &ctx->tiles_a, lb.data(), lb.size()))) {
             return rc;
@@ -1006,13 +1066,10 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
             return rc;
         }
     }
-    if ((rc = upload(ctx, &ctx->tile_src, ts.data(), ts.size()))) {
+    if ((rc = upload(ctx, &ctx->tiles, meta.data(), meta.size()))) {
         return rc;
     }
-    if ((rc = upload(ctx, &ctx->tile_rec_ptr, ptr.data(), ptr.size()))) {
-        return rc;
-    }
-    return upload(ctx, &ctx->tile_rec_idx, idx.data(), idx.size());
+    return upload(ctx, &ctx->tile_rec, recs.data(), recs.size());
 }
 
 KArgs make_args(const mbh_ctx* ctx, int in_buf, uint64_t n_off,
@@ -1045,8 +1102,11 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
     std::vector<uint32_t> cs;
     /* cells per lane (tiles of several wavefronts count as their cells
      * per lane of the first) */
+    const bool one_cell = ctx->form == MBH_FORM_MFMA ||
+        ctx->form == MBH_FORM_MFMA64; /* tiles of 64 cells only */
     for (uint32_t C : { 1u, 2u, 4u, 8u, 16u }) {
-        if (find_kernel(ctx->algo, ctx->levels, kform, C, ctx->order) &&
+        if ((C == 1u || !one_cell) &&
+            find_kernel(ctx->algo, ctx->levels, kform, C, ctx->order) &&
             (!req_tile || req_tile == 64u * C)) {
             cs.push_back(C);
         }
@@ -1191,10 +1251,10 @@ KArgs make_args(const mbh_ctx* ctx, int in_buf, uint64_t n_off,
     k.qstride = ctx->qstride;
     k.yshift = yshift(ctx);
     k.src = ctx->src;
-    k.tile_src = ctx->tile_src;
-    k.rec = ctx->rec;
-    k.tile_rec_ptr = ctx->tile_rec_ptr;
-    k.tile_rec_idx = ctx->tile_rec_idx;
+    k.tiles = ctx->tiles;
+    k.src_data = ctx->src_data;
+    k.n_t = ctx->n_t;
+    k.tile_rec = ctx->tile_rec;
     k.n_base = ctx->n_base;
     k.n_off = n_off;
     k.nsteps = nsteps;
@@ -1420,11 +1480,13 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
     std::vector<int32_t> mat(G, -1);
     std::vector<uint8_t> hz(G, 1);
     std::vector<double> fdtd((size_t)nmat_total * FDTD_STRIDE);
-    /* the device copy of a z-form blob gets y* appended (OFF_YEQ) */
+    /* the device copy of a z-form blob gets y* (OFF_YEQ) and the rows of the
+     * populations (OFF_POP) appended */
     const uint64_t src_stride =
         c->zform ? runs[0].zform_stride : runs[0].qm_stride;
     c->qstride = c->bloch ? BLOCH2_STRIDE
-                          : (c->zform ? src_stride + c->dref : src_stride);
+                          : (c->zform ? zform_stride_dev(c->levels)
+                                      : src_stride);
     if (c->planes) {
         c->qstride = rodrp_stride(c->levels);
     }
@@ -1457,6 +1519,7 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
                             src_stride * sizeof(double));
                 if (c->zform) {
                     zform_yeq(c->levels, dst, dst + src_stride);
+                    zform_pop(c->levels, dst, dst + src_stride + c->dref);
                 }
             }
         }
@@ -1464,15 +1527,18 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
     }
 
     if (c->bloch) {
-        /* algo_bloch2r: beta_y, d alpha0 / d e and the p coefficients of
-         * tau and m_z exactly zero in every material with a density, and
-         * every material lossless (fac_a exactly 1) */
+        /* algo_bloch2r: beta_x at e = 0, d beta_z / d e, beta_y,
+         * d alpha0 / d e and the p coefficients of tau and m_z exactly zero
+         * and the trace kept in every material with a density, and every
+         * material lossless (fac_a exactly 1) */
         c->bloch_real = true;
         for (size_t mi = 0; mi + BLOCH2_STRIDE <= qm.size();
              mi += BLOCH2_STRIDE) {
             const double* o = &qm[mi];
-            if (o[0] != 0.0 && (o[2] != 0.0 || o[5] != 0.0 || o[8] != 0.0 ||
-                                o[14] != 0.0 || o[17] != 0.0)) {
+            if (o[0] != 0.0 &&
+                (o[1] != 0.0 || o[2] != 0.0 || o[5] != 0.0 || o[6] != 0.0 ||
+                 o[8] != 0.0 || o[14] != 0.0 || o[17] != 0.0 ||
+                 o[10] != 1.0 || o[11] != 0.0)) {
                 c->bloch_real = false;
             }
         }
@@ -1522,11 +1588,22 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
         }                                                                     \
     } while (0)
 
-    RC(upload(c, &c->mat, mat.data(), mat.size()));
+    {
+        /* the device copy carries each cell's density flag */
+        std::vector<int32_t> mq(mat);
+        if (c->qstride) {
+            for (int32_t& v : mq) {
+                if (v >= 0 && qm[(size_t)v * c->qstride] != 0.0) {
+                    v |= MAT_QM;
+                }
+            }
+        }
+        RC(upload(c, &c->mat, mq.data(), mq.size()));
+    }
     RC(upload(c, &c->hzero, hz.data(), hz.size()));
     RC(upload(c, &c->fdtd, fdtd.data(), fdtd.size()));
     RC(upload(c, &c->qm, qm.data(), qm.size()));
-    if (c->form == MBH_FORM_MFMA || c->form == MBH_FORM_MFMA64) {
+    if (on_matrix_cores(c->levels, c->form)) {
         const uint64_t nm = qm.size() / std::max<uint64_t>(1, c->qstride);
         c->frag_stride = zm_bytes(c->levels);
         std::vector<unsigned char> fr(nm * c->frag_stride);
@@ -1653,26 +1730,32 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
             total += (uint64_t)runs[r].num_sources * c->n_t;
         }
         RC(dalloc(c, (void**)&c->src_data, total * sizeof(double)));
-        uint64_t off = 0;
+        std::vector<std::pair<uint64_t, const double*>> order;
         for (uint32_t r = 0; r < num_runs; r++) {
             const mbh_problem& p = runs[r];
             for (uint32_t k = 0; k < p.num_sources; k++) {
-                HIP_TRY(c, hipMemcpy(c->src_data + off,
-                                     p.source_data + (size_t)k * c->n_t,
-                                     c->n_t * sizeof(double),
-                                     hipMemcpyHostToDevice));
                 dev_source s{};
                 s.gx = c->runs[r].base + p.sources[k].x_idx;
-                s.data = c->src_data + off;
                 s.type = p.sources[k].type;
                 c->srcs.push_back(s);
-                off += c->n_t;
+                order.emplace_back(s.gx,
+                                   p.source_data + (size_t)k * c->n_t);
             }
         }
         std::stable_sort(c->srcs.begin(), c->srcs.end(),
                          [](const dev_source& a, const dev_source& b) {
                              return a.gx < b.gx;
                          });
+        std::stable_sort(order.begin(), order.end(),
+                         [](const std::pair<uint64_t, const double*>& a,
+                            const std::pair<uint64_t, const double*>& b) {
+                             return a.first < b.first;
+                         });
+        for (size_t i = 0; i < order.size(); i++) {
+            HIP_TRY(c, hipMemcpy(c->src_data + i * c->n_t, order[i].second,
+                                 c->n_t * sizeof(double),
+                                 hipMemcpyHostToDevice));
+        }
         RC(upload(c, &c->src, c->srcs.data(), c->srcs.size()));
     }
 
@@ -1701,7 +1784,6 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
                 c->recs.push_back(d);
             }
         }
-        RC(upload(c, &c->rec, c->recs.data(), c->recs.size()));
     }
 
     RC(dalloc(c, (void**)&c->n_base, sizeof(uint64_t)));
@@ -1710,7 +1792,7 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
 
     /* MFMA form: the tile list puts tiles with more than one material
      * (VALU path inside the kernel) first */
-    if (c->form == MBH_FORM_MFMA || c->form == MBH_FORM_MFMA64) {
+    if (on_matrix_cores(c->levels, c->form)) {
         c->split = true;
         c->mat_h = mat;
         c->mat_has_qm.resize(qm.size() / std::max<uint64_t>(1, c->qstride));

@@ -15,6 +15,7 @@
 
 #include <hip/hip_runtime.h>
 #include <type_traits>
+#include <utility>
 #include <stdint.h>
 
 #include "../../include/mbsolve_hip.h"
@@ -162,10 +163,79 @@ __device__ __forceinline__ void cinverse(const cplx* A, cplx* R)
     }
 }
 
+/* NC constants of one material, the same for every lane, sixteen to a
+ * register pair: lane l of each row of 16 lanes holds constants
+ * 16 i + l % 16, and v_fmac_f64 with DPP row_newbcast multiplies by one of
+ * them.  An FMA with such a constant then takes no load and no further
+ * instruction, where scalar loads or LDS reads of some hundred constants
+ * stall every step of a grid that leaves one wavefront on a SIMD.  (Measured
+ * on one wavefront per SIMD: every VALU instruction issues 5 cycles after the
+ * one before, a dependent FP64 FMA too, one with DPP after 6.)
+ * All lanes must be active: an FMA reads the row's other lanes.
+ * DPP reads a register no earlier than two wait states after its write.
+ * The registers are written by loads before the steps; pin() at the start of
+ * a step keeps those states where the compiler copies one (nothing else
+ * writes them, and no kernel that uses them spills). */
+template<int NC>
+struct row_consts {
+    static constexpr int NR = (NC + 15) / 16;
+    double r[NR];
+
+    __device__ __forceinline__ void load(const double* p)
+    {
+        const int l = threadIdx.x & 15;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            r[i] = p[16 * i + l < NC ? 16 * i + l : NC - 1];
+        }
+    }
+    __device__ __forceinline__ void pin()
+    {
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            asm volatile("" : "+v"(r[i]));
+        }
+        asm volatile("s_nop 1" : "+v"(r[NR - 1]));
+    }
+    /* acc += constant I * x */
+    template<int I>
+    __device__ __forceinline__ void fmac(double& acc, double x) const
+    {
+        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf "
+            "bank_mask:0xf"
+            : "+v"(acc)
+            : "v"(r[I / 16]), "v"(x), "n"(I % 16));
+    }
+    /* constant I in every lane */
+    template<int I>
+    __device__ __forceinline__ double get() const
+    {
+        return __longlong_as_double(__builtin_amdgcn_update_dpp(
+            0ll, __double_as_longlong(r[I / 16]), 0x150 + I % 16, 0xf, 0xf,
+            true));
+    }
+};
+
+/* calls f(std::integral_constant<int, i>()) for i = 0 .. N - 1 */
+template<typename F, int... I>
+__device__ __forceinline__ void static_for(F&& f,
+                                           std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>()), ...);
+}
+template<int N, typename F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for(f, std::make_integer_sequence<int, N>());
+}
+
 /* ======================================================================
  * lindblad_noop (algo_lindblad_noop.hpp:35-86): no density, p untouched.
  * ==================================================================== */
 struct algo_noop {
+    static constexpr int ROWC_WAVES = 1;
+    static constexpr bool CONSTS = false;
+    static constexpr bool ROWC = false;
     static constexpr int STAGE = 0;
     static constexpr bool SHIFT = false;
     static constexpr bool FAST_FDTD = false;
@@ -205,6 +275,9 @@ struct algo_noop_hz0 : algo_noop_fast {};
  * ==================================================================== */
 template<int N>
 struct algo_cayley {
+    static constexpr int ROWC_WAVES = 1;
+    static constexpr bool CONSTS = false;
+    static constexpr bool ROWC = false;
     static constexpr int STAGE = 0;
     static constexpr bool SHIFT = false;
     static constexpr bool FAST_FDTD = false;
@@ -374,9 +447,11 @@ struct algo_cayley {
  *   [14..17] p = P . (tau, m_x, m_y, m_z)
  *   [18..21] populations: rho00 = R00 tau + R01 m_z, rho11 = R10 tau + R11 m_z
  *   [22..25] D1 (row-major)  [26] g  [27] 1 + alpha0^2 at e = 0
+ *   [28] (beta_z at e = 0)^2
  * ==================================================================== */
 template<bool REAL>
 struct algo_bloch2_t {
+    static constexpr int ROWC_WAVES = 1;
     static constexpr int STAGE = 0;
     static constexpr bool SHIFT = false;
     static constexpr int DC = 4;
@@ -388,108 +463,123 @@ struct algo_bloch2_t {
 
     __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
-    /* 2 / n2 for n2 near 1: hardware reciprocal and two Newton steps */
-    __device__ static double two_over(double n2)
+    /* Constants of one material, loaded before the steps of a launch: from
+     * a wave-uniform address they stay in SGPRs (read inside the step they
+     * cost two scalar-load latencies per step), from a lane's own address
+     * (one cell per lane) in VGPRs, so that every lane updates with its own
+     * material's constants and no step has a branch on the material.
+     * one(): a medium without a density, which leaves the state as it is
+     * and p at zero. */
+    static constexpr bool CONSTS = true;
+    static constexpr bool ROWC = false;
+    struct consts {
+        double bcx, bcy, bcz, bex, bey, bez, a0c, a0e, g2;
+        double F00, F01, F10, F11, P0, P1, P2, P3;
+        double bz2, A0; /* REAL: bcz^2, 1 + a0c^2 */
+    };
+    template<typename P>
+    __device__ static consts load(P q)
     {
-        double r = __builtin_amdgcn_rcp(n2);
-        double t = fma(-n2, r, 1.0);
-        r = fma(r, t, r);
-        t = fma(-n2, r, 1.0);
-        r = fma(r, t, r);
-        return 2.0 * r;
+        consts k;
+        k.bcx = q[1];
+        k.bcy = q[2];
+        k.bcz = q[3];
+        k.bex = q[4];
+        k.bey = q[5];
+        k.bez = q[6];
+        k.a0c = q[7];
+        k.a0e = q[8];
+        k.g2 = q[9];
+        k.F00 = q[10];
+        k.F01 = q[11];
+        k.F10 = q[12];
+        k.F11 = q[13];
+        k.P0 = q[14];
+        k.P1 = q[15];
+        k.P2 = q[16];
+        k.P3 = q[17];
+        k.bz2 = q[28];
+        k.A0 = q[27];
+        return k;
+    }
+    __device__ static consts one()
+    {
+        consts k{};
+        k.g2 = k.F00 = k.F11 = k.A0 = 1.0;
+        return k;
     }
 
-    template<int C>
-    __device__ static void update_multi(cdp q, state* s, const double* e,
-                                        double* p)
+    /* 2 / n2 for n2 near 1: hardware reciprocal and one cubic step (with
+     * t = 1 - n2 r of at most 2^-20, r (1 + t + t^2) is off by t^3 / 2) */
+    __device__ static double two_over(double n2)
     {
-        if constexpr (REAL) {
-            update_real<C>(q, s, e, p);
-            return;
-        }
-        const double bcx = q[1], bcy = q[2], bcz = q[3];
-        const double bex = q[4], bey = q[5], bez = q[6];
-        const double a0c = q[7], a0e = q[8], g2 = q[9];
-        const double F00 = q[10], F01 = q[11], F10 = q[12], F11 = q[13];
-        const double P0 = q[14], P1 = q[15], P2 = q[16], P3 = q[17];
+        const double r = __builtin_amdgcn_rcp(n2);
+        const double t = fma(-n2, r, 1.0);
+        const double u = fma(r, fma(t, t, t), r);
+        return u + u;
+    }
+
+    /* C cells of one material.  The rotation is written with
+     * c = beta x m and u = lambda (s m + c):  m' = m + beta x u, whose y
+     * component expands to m_y + lambda (s c_y + beta_y (beta.m) -
+     * |beta|^2 m_y).
+     * REAL: beta_y, d alpha0 / d e and the p coefficients of tau and m_z
+     * are exactly zero, so are beta_x at e = 0 and d beta_z / d e (a
+     * diagonal Hamiltonian and a real off-diagonal dipole, as qm_desc_2lvl
+     * builds them, qm_description.hpp:338-432), and F00 = 1, F01 = 0 (the
+     * relaxation keeps the trace).  The terms dropped are exact zeros and
+     * ones of the general form, so the results are the same (up to the sign
+     * of zeros): 24 FP64 instructions per cell where the general form takes
+     * about 45. */
+    template<int C>
+    __device__ static void apply(const consts& k, state* s, const double* e,
+                                 double* p)
+    {
 #pragma unroll
         for (int c = 0; c < C; c++) {
             double* v = s[c].v;
             /* second half step of the previous step and first half step
              * of this one */
-            const double tr = fma(F01, v[3], F00 * v[0]);
-            const double mz = fma(F11, v[3], F10 * v[0]);
-            const double mx = g2 * v[1];
-            const double my = g2 * v[2];
+            const double tr = REAL ? v[0] : fma(k.F01, v[3], k.F00 * v[0]);
+            const double mz = fma(k.F11, v[3], k.F10 * v[0]);
+            const double mx = k.g2 * v[1];
+            const double my = k.g2 * v[2];
             /* Cayley rotation at field e */
-            const double bx = fma(e[c], bex, bcx);
-            const double by = fma(e[c], bey, bcy);
-            const double bz = fma(e[c], bez, bcz);
-            const double a0 = fma(e[c], a0e, a0c);
-            const double r2 = fma(bz, bz, fma(by, by, bx * bx));
-            const double sc = fma(-0.25, r2, fma(a0, a0, 1.0));
+            const double bx =
+                REAL ? e[c] * k.bex : fma(e[c], k.bex, k.bcx);
+            const double by = REAL ? 0.0 : fma(e[c], k.bey, k.bcy);
+            const double bz = REAL ? k.bcz : fma(e[c], k.bez, k.bcz);
+            const double r2 =
+                REAL ? fma(bx, bx, k.bz2) : fma(bx, bx, fma(by, by, bz * bz));
+            const double a0 = REAL ? 0.0 : fma(e[c], k.a0e, k.a0c);
+            const double sc = fma(-0.25, r2, REAL ? k.A0 : fma(a0, a0, 1.0));
             const double lam = two_over(fma(sc, sc, r2));
-            const double c1x = fma(by, mz, -(bz * my));
-            const double c1y = fma(bz, mx, -(bx * mz));
-            const double c1z = fma(bx, my, -(by * mx));
-            const double bm = fma(bz, mz, fma(by, my, bx * mx));
-            const double c2x = fma(bx, bm, -(mx * r2));
-            const double c2y = fma(by, bm, -(my * r2));
-            const double c2z = fma(bz, bm, -(mz * r2));
+            const double cy = fma(bz, mx, -(bx * mz));
+            const double uy = lam * fma(sc, my, cy);
             v[0] = tr;
-            v[1] = fma(lam, fma(sc, c1x, c2x), mx);
-            v[2] = fma(lam, fma(sc, c1y, c2y), my);
-            v[3] = fma(lam, fma(sc, c1z, c2z), mz);
-            p[c] = fma(P3, v[3], fma(P2, v[2], fma(P1, v[1], P0 * tr)));
-        }
-    }
-
-    /* The same step for a material whose beta_y, d alpha0 / d e and the
-     * p coefficients of tau and m_z are exactly zero (a diagonal
-     * Hamiltonian and a real off-diagonal dipole, as qm_desc_2lvl builds
-     * them, qm_description.hpp:338-432): those terms are dropped and
-     * 1 + alpha0^2 is the blob's [27].  Each dropped term is an exact zero
-     * in the general form, so the results are the same (up to the sign of
-     * zeros). */
-    template<int C>
-    __device__ static void update_real(cdp q, state* s, const double* e,
-                                       double* p)
-    {
-        const double bcx = q[1], bcz = q[3];
-        const double bex = q[4], bez = q[6];
-        const double A0 = q[27], g2 = q[9];
-        const double F00 = q[10], F01 = q[11], F10 = q[12], F11 = q[13];
-        const double P1 = q[15], P2 = q[16];
-#pragma unroll
-        for (int c = 0; c < C; c++) {
-            double* v = s[c].v;
-            const double tr = fma(F01, v[3], F00 * v[0]);
-            const double mz = fma(F11, v[3], F10 * v[0]);
-            const double mx = g2 * v[1];
-            const double my = g2 * v[2];
-            const double bx = fma(e[c], bex, bcx);
-            const double bz = fma(e[c], bez, bcz);
-            const double r2 = fma(bz, bz, bx * bx);
-            const double sc = fma(-0.25, r2, A0);
-            const double lam = two_over(fma(sc, sc, r2));
-            const double c1x = -(bz * my);
-            const double c1y = fma(bz, mx, -(bx * mz));
-            const double c1z = bx * my;
-            const double bm = fma(bz, mz, bx * mx);
-            const double c2x = fma(bx, bm, -(mx * r2));
-            const double c2y = -(my * r2);
-            const double c2z = fma(bz, bm, -(mz * r2));
-            v[0] = tr;
-            v[1] = fma(lam, fma(sc, c1x, c2x), mx);
-            v[2] = fma(lam, fma(sc, c1y, c2y), my);
-            v[3] = fma(lam, fma(sc, c1z, c2z), mz);
-            p[c] = fma(P2, v[2], P1 * v[1]);
+            if constexpr (REAL) {
+                v[1] = fma(-bz, uy, mx);
+                v[3] = fma(bx, uy, mz);
+                v[2] = fma(lam, fma(sc, cy, -(r2 * my)), my);
+                p[c] = fma(k.P2, v[2], k.P1 * v[1]);
+            } else {
+                const double cx = fma(by, mz, -(bz * my));
+                const double cz = fma(bx, my, -(by * mx));
+                const double ux = lam * fma(sc, mx, cx);
+                const double uz = lam * fma(sc, mz, cz);
+                const double bm = fma(bz, mz, fma(by, my, bx * mx));
+                v[1] = fma(by, uz, fma(-bz, uy, mx));
+                v[3] = fma(-by, ux, fma(bx, uy, mz));
+                v[2] = fma(lam, fma(sc, cy, fma(by, bm, -(r2 * my))), my);
+                p[c] = fma(k.P3, v[3],
+                           fma(k.P2, v[2], fma(k.P1, v[1], k.P0 * tr)));
+            }
         }
     }
 
     __device__ static void update(cdp q, state& s, double e, double& p)
     {
-        update_multi<1>(q, &s, &e, &p);
+        apply<1>(load(q), &s, &e, &p);
     }
 
     __device__ static double population(cdp q, const state& s, int m)
@@ -532,16 +622,11 @@ __device__ __forceinline__ double cv_population(const double* d, int m)
         double sum = 0.0;
 #pragma unroll
         for (int i = 0; i < N - 1; i++) {
-            double factor;
-            if (m < i + 1) {
-                factor = -1.0;
-            } else if (m == i + 1) {
-                factor = (double)m;
-            } else {
-                factor = 0.0;
-            }
-            int k = ((i + 1) * (i + 2)) / 2;
-            sum += factor / sqrt((double)k) * d[N * (N - 1) + i];
+            /* -1, m or 0 over sqrt(k), folded: no division at run time */
+            const double root = sqrt((double)(((i + 1) * (i + 2)) / 2));
+            const double below = -1.0 / root, at = (double)(i + 1) / root;
+            const double f = m < i + 1 ? below : (m == i + 1 ? at : 0.0);
+            sum += f * d[N * (N - 1) + i];
         }
         return 1.0 / N + 0.5 * sum;
     }
@@ -556,6 +641,9 @@ __device__ __forceinline__ double cv_population(const double* d, int m)
  * ==================================================================== */
 template<int N>
 struct algo_rodr {
+    static constexpr int ROWC_WAVES = 1;
+    static constexpr bool CONSTS = false;
+    static constexpr bool ROWC = false;
     static constexpr int STAGE = 0;
     static constexpr bool SHIFT = false;
     static constexpr bool FAST_FDTD = false;
@@ -764,6 +852,19 @@ __device__ __forceinline__ void tier_sincos(double x, double& s, double& c)
         s = fma(x * x2, fma(x2, 8.3333333333333333333e-03,
                             -1.6666666666666666667e-01), x);
         c = fma(x2, fma(x2, 4.1666666666666666667e-02, -0.5), 1.0);
+    } else if constexpr (TIER == 4) {
+        /* |x| <= 2^-5: to x^9 / x^8 (below 1e-22) */
+        const double x2 = x * x;
+        double ps = fma(x2, 2.7557319223985890653e-06,
+                        -1.9841269841269841270e-04);
+        ps = fma(ps, x2, 8.3333333333333333333e-03);
+        ps = fma(ps, x2, -1.6666666666666666667e-01);
+        s = fma(x * x2, ps, x);
+        double pc = fma(x2, 2.4801587301587301587e-05,
+                        -1.3888888888888888889e-03);
+        pc = fma(pc, x2, 4.1666666666666666667e-02);
+        pc = fma(pc, x2, -0.5);
+        c = fma(pc, x2, 1.0);
     } else if constexpr (TIER == 2) {
         taylor_sincos(x, s, c);
     } else {
@@ -804,9 +905,7 @@ __device__ __forceinline__ void tier_sincos(double x, double& s, double& c)
  * |x| <= 0.25 (to x^13 / x^14); else the library. */
 constexpr double PLANE_SMALL = 0.03125;
 
-__device__ __forceinline__ void plane_sincos(double x, bool small, bool medium,
-                                             bool all_small, bool all_medium,
-                                             double& s, double& v)
+__device__ __forceinline__ void plane_small(double x, double& s, double& v)
 {
     const double x2 = x * x;
     double ps = 2.7557319223985890653e-06;        /* 1/9! */
@@ -819,41 +918,49 @@ __device__ __forceinline__ void plane_sincos(double x, bool small, bool medium,
     pc = fma(pc, x2, -4.1666666666666666667e-02); /* -1/4! */
     pc = fma(pc, x2, 0.5);                        /* 1/2! */
     v = pc * x2;
-    if (!all_small) {
-        double qs = 1.6059043836821614599e-10;        /* 1/13! */
-        qs = fma(qs, x2, -2.5052108385441718775e-08); /* -1/11! */
-        qs = fma(qs, x2, 2.7557319223985890653e-06);
-        qs = fma(qs, x2, -1.9841269841269841270e-04);
-        qs = fma(qs, x2, 8.3333333333333333333e-03);
-        qs = fma(qs, x2, -1.6666666666666666667e-01);
-        double s2 = fma(qs * x2, x, x);
-        double qc = 1.1470745597729724714e-11;        /* 1/14! */
-        qc = fma(qc, x2, -2.0876756987868098979e-09); /* -1/12! */
-        qc = fma(qc, x2, 2.7557319223985890653e-07);  /* 1/10! */
-        qc = fma(qc, x2, -2.4801587301587301587e-05);
-        qc = fma(qc, x2, 1.3888888888888888889e-03);
-        qc = fma(qc, x2, -4.1666666666666666667e-02);
-        qc = fma(qc, x2, 0.5);
-        double v2 = qc * x2;
-        if (!all_medium) {
-            double sl, cl;
-            sincos(x, &sl, &cl);
-            s2 = medium ? s2 : sl;
-            v2 = medium ? v2 : 1.0 - cl;
-        }
-        s = small ? s : s2;
-        v = small ? v : v2;
+}
+
+__device__ __forceinline__ void plane_sincos(double x, bool small, bool medium,
+                                             bool all_medium, double& s,
+                                             double& v)
+{
+    plane_small(x, s, v);
+    const double x2 = x * x;
+    double qs = 1.6059043836821614599e-10;        /* 1/13! */
+    qs = fma(qs, x2, -2.5052108385441718775e-08); /* -1/11! */
+    qs = fma(qs, x2, 2.7557319223985890653e-06);
+    qs = fma(qs, x2, -1.9841269841269841270e-04);
+    qs = fma(qs, x2, 8.3333333333333333333e-03);
+    qs = fma(qs, x2, -1.6666666666666666667e-01);
+    double s2 = fma(qs * x2, x, x);
+    double qc = 1.1470745597729724714e-11;        /* 1/14! */
+    qc = fma(qc, x2, -2.0876756987868098979e-09); /* -1/12! */
+    qc = fma(qc, x2, 2.7557319223985890653e-07);  /* 1/10! */
+    qc = fma(qc, x2, -2.4801587301587301587e-05);
+    qc = fma(qc, x2, 1.3888888888888888889e-03);
+    qc = fma(qc, x2, -4.1666666666666666667e-02);
+    qc = fma(qc, x2, 0.5);
+    double v2 = qc * x2;
+    if (!all_medium) {
+        double sl, cl;
+        sincos(x, &sl, &cl);
+        s2 = medium ? s2 : sl;
+        v2 = medium ? v2 : 1.0 - cl;
     }
+    s = small ? s : s2;
+    v = small ? v : v2;
 }
 
 template<int N>
 struct algo_rodrp {
+    static constexpr bool CONSTS = false;
     static constexpr bool SHIFT = false;
     static constexpr bool FAST_FDTD = false;
     static constexpr int K = N * N - 1;
     static constexpr int B = K / 2;
     static constexpr int DC = K;
     static constexpr int STATE = K;
+    static constexpr int ROWC_WAVES = 2;
     struct state {
         double v[STATE];
     };
@@ -865,9 +972,7 @@ struct algo_rodrp {
     static constexpr int PLANE = 1 + 2 * K;
     static constexpr int STRIDE = OFF_PL + B * PLANE;
 
-    /* three levels: the 155 constants are staged in LDS (they do not fit
-     * the SGPRs), as for the z-form */
-    static constexpr int STAGE = (K <= 8) ? STRIDE : 0;
+    static constexpr int STAGE = 0;
 
     __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
@@ -970,21 +1075,19 @@ struct algo_rodrp {
                 double u1[C], u2[C];
 #pragma unroll
                 for (int c = 0; c < C; c++) {
-                    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+                    double al = 0.0, be = 0.0;
 #pragma unroll
                     for (int k = 0; k < K; k++) {
-                        if (k & 1) {
-                            a1 = fma(q1[k], d[c][k], a1);
-                            b1 = fma(q2[k], d[c][k], b1);
-                        } else {
-                            a0 = fma(q1[k], d[c][k], a0);
-                            b0 = fma(q2[k], d[c][k], b0);
-                        }
+                        al = fma(q1[k], d[c][k], al);
+                        be = fma(q2[k], d[c][k], be);
                     }
-                    const double al = a0 + a1, be = b0 + b1;
                     double sn, vc;
-                    plane_sincos(pl[0] * e[c], small[c], medium[c], all_s,
-                                 all_m, sn, vc);
+                    if (all_s) {
+                        plane_small(pl[0] * e[c], sn, vc);
+                    } else {
+                        plane_sincos(pl[0] * e[c], small[c], medium[c],
+                                     all_m, sn, vc);
+                    }
                     u1[c] = fma(-sn, be, -(vc * al));
                     u2[c] = fma(sn, al, -(vc * be));
                 }
@@ -1001,18 +1104,112 @@ struct algo_rodrp {
         const P pv = q + OFF_PV;
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            double p0 = q[2], p1 = 0.0;
+            double acc = q[2];
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 s[c].v[k] = d[c][k];
-                if (k & 1) {
-                    p1 = fma(pv[k], d[c][k], p1);
-                } else {
-                    p0 = fma(pv[k], d[c][k], p0);
-                }
+                acc = fma(pv[k], d[c][k], acc);
             }
-            p[c] = p0 + p1;
+            p[c] = acc;
         }
+    }
+
+    /* one cell per lane, three levels: the same step with the constants
+     * from row registers (more levels would spill) */
+    static constexpr bool ROWC = N == 3;
+    static constexpr int NC = STRIDE - OFF_C;
+    struct rowc {
+        row_consts<NC> k;
+        double th[B], thmax, pb;
+        int np;
+        cdp q;
+        __device__ void load(cdp qs, const double* q)
+        {
+            this->q = qs;
+            k.load(q + OFF_C);
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                th[b] = q[OFF_PL + b * PLANE];
+            }
+            pb = q[2];
+            thmax = q[3];
+            np = (int)qs[1];
+        }
+    };
+    __device__ __forceinline__ static void rows_half(const rowc& R, const double* d, double* o)
+    {
+        static_for<K>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            double acc = R.k.template get<i>();
+            static_for<K>([&](auto k_) __attribute__((always_inline)) {
+                constexpr int kk = decltype(k_)::value;
+                R.k.template fmac<2 * K + i * K + kk>(acc, d[kk]);
+            });
+            o[i] = acc;
+        });
+    }
+    __device__ __forceinline__ static void apply_rows(rowc& R, state& s, double e, double& p,
+                                      bool mine)
+    {
+        R.k.pin();
+        double d[K], r[K];
+        rows_half(R, s.v, d);
+        const double xm = R.thmax * fabs(e);
+        const bool small = xm <= PLANE_SMALL, medium = xm <= TAYLOR_MAX;
+        const bool all_s = __all(small || !mine);
+        const bool all_m = __all(medium || !mine);
+        /* the wide ranges of the angle in a rolled loop (one copy of the
+         * library function; unrolled, its registers would halve the
+         * wavefronts per SIMD) */
+        double sn[B], vc[B];
+        if (all_s) {
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                plane_small(R.th[b] * e, sn[b], vc[b]);
+            }
+        } else {
+            double ws[B], wv[B];
+#pragma unroll 1
+            for (int b = 0; b < B; b++) {
+                plane_sincos(R.q[OFF_PL + b * PLANE] * e, small, medium,
+                             all_m, ws[b], wv[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                sn[b] = ws[b];
+                vc[b] = wv[b];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            r[k] = d[k];
+        }
+        static_for<B>([&](auto b_) __attribute__((always_inline)) {
+            constexpr int b = decltype(b_)::value;
+            constexpr int Q1 = 2 * K + K * K + b * PLANE + 1, Q2 = Q1 + K;
+            if (b < R.np) {
+                double al = 0.0, be = 0.0;
+                static_for<K>([&](auto k_) __attribute__((always_inline)) {
+                    constexpr int kk = decltype(k_)::value;
+                    R.k.template fmac<Q1 + kk>(al, d[kk]);
+                    R.k.template fmac<Q2 + kk>(be, d[kk]);
+                });
+                const double u1 = fma(-sn[b], be, -(vc[b] * al));
+                const double u2 = fma(sn[b], al, -(vc[b] * be));
+                static_for<K>([&](auto k_) __attribute__((always_inline)) {
+                    constexpr int kk = decltype(k_)::value;
+                    R.k.template fmac<Q2 + kk>(r[kk], u2);
+                    R.k.template fmac<Q1 + kk>(r[kk], u1);
+                });
+            }
+        });
+        rows_half(R, r, s.v);
+        double acc = R.pb;
+        static_for<K>([&](auto k_) __attribute__((always_inline)) {
+            constexpr int kk = decltype(k_)::value;
+            R.k.template fmac<K + kk>(acc, s.v[kk]);
+        });
+        p = acc;
     }
 
     template<int C>
@@ -1043,6 +1240,8 @@ struct algo_rodrp {
  * ==================================================================== */
 template<int N>
 struct algo_zform {
+    static constexpr int ROWC_WAVES = N <= 3 ? 3 : 2;
+    static constexpr bool CONSTS = false;
     static constexpr bool FAST_FDTD = true;
     static constexpr int K = N * N - 1;
     static constexpr int B = K / 2;
@@ -1067,6 +1266,10 @@ struct algo_zform {
      * y - y*, so its rounding scales with the distance from equilibrium
      * instead of with |y*|. */
     static constexpr int OFF_YEQ = OFF_DIN + K;
+    /* and, for the records, the populations as linear forms of y:
+     * rho_mm = r_m . y + o_m, N rows of (r_m, o_m) */
+    static constexpr int OFF_POP = OFF_YEQ + K;
+    static constexpr int DEV_STRIDE = OFF_POP + N * (K + 1);
     static constexpr bool SHIFT = true;
 
     __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
@@ -1146,8 +1349,7 @@ struct algo_zform {
                 r[c][2 * b + 1] = fma(sn[c][b], y0, cs[c][b] * y1);
             }
         }
-        /* p = a . r + b, two interleaved partial sums (shorter chain on
-         * the step's critical path) */
+        /* p = a . r + b, two interleaved partial sums */
         double pa[C], pb[C];
 #pragma unroll
         for (int c = 0; c < C; c++) {
@@ -1221,6 +1423,90 @@ struct algo_zform {
         update_multi<1>(q, &s, &e, &p);
     }
 
+    /* one cell per lane, three and four levels: the same step with W, c and
+     * a from row registers (five levels would spill at two wavefronts per
+     * SIMD) */
+    static constexpr bool ROWC = N == 3 || N == 4;
+    static constexpr int NC = K * K + 2 * K;
+    struct rowc {
+        row_consts<NC> k; /* W, c, a */
+        double th[B], thmax, b;
+        cdp q;
+        __device__ void load(cdp qs, const double* q)
+        {
+            this->q = qs;
+            k.load(q + OFF_W);
+            thmax = 0.0;
+#pragma unroll
+            for (int i = 0; i < B; i++) {
+                th[i] = q[OFF_TH + i];
+                thmax = fmax(thmax, fabs(th[i]));
+            }
+            b = q[2];
+        }
+    };
+    __device__ __forceinline__ static void apply_rows(rowc& R, state& s, double e, double& p,
+                                      bool mine)
+    {
+        R.k.pin();
+        double sn[B], cs[B], r[K];
+        /* wave-uniform tier, as in update_multi_p; the ranges beyond 2^-5 in
+         * a rolled loop (one copy of the library function; unrolled, its
+         * registers would halve the wavefronts per SIMD) */
+        const double xm = mine ? R.thmax * fabs(e) : 0.0;
+        auto tier = [&](auto t) {
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                tier_sincos<decltype(t)::value>(R.th[b] * e, sn[b], cs[b]);
+            }
+        };
+        if (__all(xm <= 0x1p-13)) {
+            tier(std::integral_constant<int, 0>());
+        } else if (__all(xm <= 0x1p-10)) {
+            tier(std::integral_constant<int, 1>());
+        } else if (__all(xm <= 0x1p-5)) {
+            tier(std::integral_constant<int, 4>());
+        } else {
+            double ws[B], wc[B];
+#pragma unroll 1
+            for (int b = 0; b < B; b++) {
+                sincos(R.q[OFF_TH + b] * e, &ws[b], &wc[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                sn[b] = ws[b];
+                cs[b] = wc[b];
+            }
+        }
+#pragma unroll
+        for (int k = 2 * B; k < K; k++) {
+            r[k] = s.v[k];
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            const double y0 = s.v[2 * b], y1 = s.v[2 * b + 1];
+            r[2 * b] = fma(cs[b], y0, -(sn[b] * y1));
+            r[2 * b + 1] = fma(sn[b], y0, cs[b] * y1);
+        }
+        double pa = R.b, pb = 0.0;
+        static_for<K>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            R.k.template fmac<K * K + K + i>(i & 1 ? pb : pa, r[i]);
+        });
+        p = pa + pb;
+        static_for<K>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            s.v[i] = R.k.template get<K * K + i>();
+        });
+        static_for<K>([&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            static_for<K>([&](auto k_) __attribute__((always_inline)) {
+                constexpr int kk = decltype(k_)::value;
+                R.k.template fmac<i * K + kk>(s.v[i], r[kk]);
+            });
+        });
+    }
+
     /* component k of the reference coherence vector after the step */
     __device__ static double dcomp(cdp q, const state& s, int k)
     {
@@ -1242,18 +1528,13 @@ struct algo_zform {
     }
     __device__ static double population(cdp q, const state& s, int m)
     {
-        double d[K];
+        cdp r = q + OFF_POP + (uint64_t)m * (K + 1);
+        double acc = r[K];
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            d[k] = 0.0;
+        for (int j = 0; j < K; j++) {
+            acc = fma(r[j], s.v[j], acc);
         }
-        if (q[0] != 0.0) {
-#pragma unroll
-            for (int k = N * (N - 1); k < K; k++) {
-                d[k] = dcomp(q, s, k);
-            }
-        }
-        return cv_population<N>(d, m);
+        return acc;
     }
 };
 

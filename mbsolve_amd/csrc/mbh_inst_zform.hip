@@ -16,7 +16,7 @@ __global__ __launch_bounds__(64) void zform_to_y(ZArgs a)
     const uint64_t i = (uint64_t)blockIdx.x * 64 + threadIdx.x;
     const uint64_t g = a.g0 + i;
     const bool in = i < a.count;
-    const int32_t m = in ? a.mat[g] : -1;
+    const int32_t m = in ? mat_of(a.mat[g]) : -1;
     double d[K], y[K];
 #pragma unroll
     for (int j = 0; j < K; j++) {
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64) void zform_from_y(ZArgs a)
     const uint64_t i = (uint64_t)blockIdx.x * 64 + threadIdx.x;
     const uint64_t g = a.g0 + i;
     const bool in = i < a.count;
-    const int32_t m = in ? a.mat[g] : -1;
+    const int32_t m = in ? mat_of(a.mat[g]) : -1;
     typename algo_zform<N>::state s;
     double d[K];
 #pragma unroll

@@ -34,13 +34,18 @@
 namespace mbh {
 
 constexpr int FDTD_STRIDE = 5; /* fac_a fac_b fac_c gamma dx_inv */
-constexpr int BLOCH2_STRIDE = 28; /* two-level Cayley, Bloch form */
+constexpr int BLOCH2_STRIDE = 29; /* two-level Cayley, Bloch form */
 
 struct dev_source {
-    uint64_t gx;         /* super-grid cell */
-    const double* data;  /* n_t values */
+    uint64_t gx; /* super-grid cell */
     uint32_t type;
     uint32_t pad;
+};
+
+/* sources inside a tile's loaded span (halo included) and its records */
+struct tile_meta {
+    uint32_t src_lo, src_hi;
+    uint32_t rec_lo, rec_hi;
 };
 
 struct dev_record {
@@ -68,16 +73,17 @@ struct KArgs {
     uint64_t Gown;    /* cells owned by tiles: G minus the trailing pseudo
                          cell (its H is read at step 0 only) */
     uint64_t dstride; /* elements between density components */
-    const int32_t* mat;   /* [G], -1: pseudo cell */
+    const int32_t* mat;   /* [G]: material, plus MAT_QM where it has a
+                             density; -1: pseudo cell */
     const uint8_t* hzero; /* [G] */
     const double* fdtd;   /* [nmat][FDTD_STRIDE] */
     const double* qm;     /* [nmat][qstride] */
     uint64_t qstride;
-    const dev_source* src;     /* sorted by gx */
-    const uint32_t* tile_src;  /* [2*num_tiles]: [lo, hi) */
-    const dev_record* rec;
-    const uint32_t* tile_rec_ptr; /* [num_tiles + 1] */
-    const uint32_t* tile_rec_idx;
+    const tile_meta* tiles;   /* [num_tiles] */
+    const dev_source* src;    /* sorted by gx */
+    const double* src_data;   /* [sources][n_t], in the order of src */
+    uint64_t n_t;
+    const dev_record* tile_rec; /* the tiles' records, tile after tile */
     const uint64_t* n_base; /* device: first step = *n_base + n_off */
     uint64_t n_off;
     uint32_t nsteps;
@@ -89,12 +95,17 @@ struct KArgs {
     const uint32_t* tile_list; /* tiles of this launch (NULL: blockIdx) */
     /* MFMA form: the first n_mixed tiles of the list hold more than one
      * material; tile_mat[i] (i: position in the list) is the material of
-     * a uniform tile, plus TILE_MAT_QM when it has a density (NULL: the
+     * a uniform tile, plus MAT_QM when it has a density (NULL: the
      * kernel reads the cells' materials) */
     const int32_t* tile_mat;
     uint32_t n_mixed;
 };
-constexpr int32_t TILE_MAT_QM = 0x40000000;
+constexpr int32_t MAT_QM = 0x40000000;
+/* material of an entry of mat (-1: pseudo cell) */
+__host__ __device__ constexpr int32_t mat_of(int32_t v)
+{
+    return v < 0 ? -1 : (v & ~MAT_QM);
+}
 /* kernel-table forms of the specialised kernels (internal, beside the
  * MBH_FORM_*): algo_noop_hz0, and algo_bloch2r with FP32 / FP64 state */
 constexpr uint32_t KFORM_NOOP_HZ0 = 0x100;
@@ -164,10 +175,70 @@ __device__ __forceinline__ void for_each_material(int32_t m, F&& fn)
     }
 }
 
-__device__ __forceinline__ dev_record load_record(const dev_record* base,
-                                                 uint32_t i)
+/* copy_list_entry_dev::hasto_record (copy_list_entry.hpp:74-80) plus the
+ * row bound */
+__device__ __forceinline__ bool record_now(double ratio, uint64_t rows,
+                                           uint64_t n)
 {
-    const auto* r = as_const(base) + i;
+    bool now = (n == 0);
+    if (!now) {
+        now = floor(ratio * (double)(n - 1)) != floor(ratio * (double)n);
+    }
+    return now && (uint64_t)floor(ratio * (double)n) < rows;
+}
+
+/* Records of a tile.  At the start of a launch the first REC_LANES of them
+ * are evaluated for all steps of the block, one step per lane, and their
+ * rows put in an LDS table (row minus the row at the block's first step;
+ * REC_NOT: not due).  At a step with a due record lane r reads record r's
+ * entry, and each due one is handed to the whole wavefront by readlane: one
+ * LDS latency for all records of a step, where evaluating the row rule and
+ * reading the descriptors cost some 700 cycles per record and step.  The
+ * cells of a record at tile offsets [lo, hi) (clipped to the owned cells;
+ * the tile's first cell, halo included, has offset 0) go to base + 8 offset
+ * plus the row's offset.  Nothing but the table and the step mask stays live
+ * over the steps.  Records beyond REC_LANES are read from memory at every
+ * step that has one due. */
+constexpr uint32_t REC_LANES = 16;
+constexpr uint32_t REC_NOT = 0xffu;
+constexpr uint32_t REC_STEPS = 64; /* largest temporal block */
+struct rec_stage {
+    uint64_t base[REC_LANES];
+    uint64_t row_bytes[REC_LANES];
+    uint32_t span[REC_LANES]; /* lo | hi << 16 */
+    uint32_t what[REC_LANES]; /* type | level << 8 */
+    uint32_t r_lo, nrec;
+    uint32_t density; /* a population or the inversion may be among them */
+    int64_t tile0, own_lo, own_hi;
+    uint8_t row[REC_STEPS][REC_LANES];
+};
+
+/* coherences are not recorded */
+__device__ __forceinline__ bool record_skipped(const dev_record& R)
+{
+    return R.type == MBH_REC_DENSITY && R.row_idx != R.col_idx;
+}
+
+__device__ __forceinline__ uint32_t lane_u32(uint32_t x, int i)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, i);
+}
+__device__ __forceinline__ uint64_t lane_u64(uint64_t x, int i)
+{
+    return ((uint64_t)lane_u32((uint32_t)(x >> 32), i) << 32) |
+        lane_u32((uint32_t)x, i);
+}
+__device__ __forceinline__ double lane_f64(double x, int i)
+{
+    return __longlong_as_double(
+        (long long)lane_u64((uint64_t)__double_as_longlong(x), i));
+}
+
+/* record i of the launch's list through scalar loads */
+__device__ __forceinline__ dev_record scalar_record(const KArgs& k,
+                                                    uint32_t i)
+{
+    const auto* r = as_const(k.tile_rec) + i;
     dev_record R;
     R.gbegin = r->gbegin;
     R.cols = r->cols;
@@ -181,36 +252,127 @@ __device__ __forceinline__ dev_record load_record(const dev_record* base,
     return R;
 }
 
-/* copy_list_entry_dev::hasto_record (copy_list_entry.hpp:74-80) plus the
- * row bound */
-__device__ __forceinline__ bool record_now(double ratio, uint64_t rows,
-                                           uint64_t n)
+/* where record R goes at row `row`, and its span in the tile */
+__device__ __forceinline__ uint64_t record_base(const dev_record& R,
+                                                uint64_t row, int64_t tile0)
 {
-    bool now = (n == 0);
-    if (!now) {
-        now = floor(ratio * (double)(n - 1)) != floor(ratio * (double)n);
-    }
-    return now && (uint64_t)floor(ratio * (double)n) < rows;
+    return (uint64_t)(uintptr_t)R.dst + 8u * (row * R.cols) -
+        8u * (uint64_t)((int64_t)R.gbegin - tile0);
+}
+__device__ __forceinline__ uint32_t record_span(const dev_record& R,
+                                                int64_t tile0, int64_t own_lo,
+                                                int64_t own_hi)
+{
+    const int64_t g0 = (int64_t)R.gbegin, g1 = g0 + (int64_t)R.cols;
+    const uint32_t lo = (uint32_t)((g0 > own_lo ? g0 : own_lo) - tile0);
+    const uint32_t hi = (uint32_t)((g1 < own_hi ? g1 : own_hi) - tile0);
+    return lo | (hi << 16);
 }
 
-template<class A>
-__device__ __forceinline__ double record_value(const KArgs& k, uint32_t type,
-                                               uint32_t row, int32_t m,
-                                               double e, double h, double p,
-                                               const typename A::state& d)
+/* R: lane r's record r of the tile (r < REC_LANES, loaded by the caller
+ * together with the state).  Returns the steps of the block at which any of
+ * the tile's records is due (one bit per step) and, if there are any, stages
+ * them. */
+__device__ __forceinline__ uint64_t stage_records(
+    const KArgs& k, rec_stage& S, const dev_record& R, int lane, bool writer,
+    const tile_meta& M, int64_t own_lo, int64_t own_hi, uint64_t n0,
+    uint32_t nsteps)
 {
-    cdp q = (cdp)k.qm + (uint64_t)(m < 0 ? 0 : m) * k.qstride;
-    switch (type) {
-    case MBH_REC_ELECTRIC:
-        return e;
-    case MBH_REC_POLAR_DT:
-        return p;
-    case MBH_REC_MAGNETIC:
-        return h;
-    case MBH_REC_INVERSION:
-        return (m < 0 || k.qstride == 0) ? 0.0 : A::inversion(q, d);
-    default: /* density: only populations are recorded */
-        return (m < 0 || k.qstride == 0) ? 0.0 : A::population(q, d, row);
+    static_assert(REC_STEPS == 64, "one lane and one mask bit per step");
+    const uint32_t nrec = M.rec_hi - M.rec_lo;
+    const uint32_t nlane = nrec < REC_LANES ? nrec : REC_LANES;
+    const uint64_t n = n0 + (uint64_t)lane;
+    const bool step = lane < (int)nsteps;
+    uint64_t steps = 0;
+    for (uint32_t i = 0; i < nrec; i++) {
+        double ratio;
+        uint64_t rows;
+        bool skip;
+        if (i < REC_LANES) {
+            ratio = lane_f64(R.ratio, (int)i);
+            rows = lane_u64(R.rows, (int)i);
+            skip = lane_u32(record_skipped(R) ? 1u : 0u, (int)i) != 0u;
+        } else {
+            const dev_record Q = scalar_record(k, M.rec_lo + i);
+            ratio = Q.ratio;
+            rows = Q.rows;
+            skip = record_skipped(Q);
+        }
+        const bool due = step && !skip && record_now(ratio, rows, n);
+        if (i < REC_LANES && writer) {
+            const uint64_t row = (uint64_t)floor(ratio * (double)n);
+            const uint64_t row0 = (uint64_t)floor(ratio * (double)n0);
+            S.row[lane][i] =
+                due ? (uint8_t)(row - row0) : (uint8_t)REC_NOT;
+        }
+        steps |= __ballot(due);
+    }
+    if (steps != 0ull) {
+        if (writer) {
+            const int64_t tile0 = own_lo - (int64_t)k.halo;
+            const bool dens = __any((uint32_t)lane < nlane &&
+                                    !record_skipped(R) &&
+                                    R.type >= MBH_REC_DENSITY) ||
+                nrec > REC_LANES;
+            if ((uint32_t)lane < nlane) {
+                const uint64_t row0 =
+                    (uint64_t)floor(R.ratio * (double)n0);
+                S.base[lane] = record_base(R, row0, tile0);
+                S.row_bytes[lane] = 8u * R.cols;
+                S.span[lane] = record_span(R, tile0, own_lo, own_hi);
+                S.what[lane] = R.type | (R.row_idx << 8);
+            }
+            if (lane == 0) {
+                S.r_lo = M.rec_lo;
+                S.nrec = nrec;
+                S.density = dens ? 1u : 0u;
+                S.tile0 = tile0;
+                S.own_lo = own_lo;
+                S.own_hi = own_hi;
+            }
+        }
+        __syncthreads();
+    }
+    return steps;
+}
+
+/* Calls put(dst, lo, hi, type, level) for every record due at step s of the
+ * block (step n of the run), all arguments wave-uniform: the cell at tile
+ * offset o in [lo, hi) goes to dst[o]. */
+template<typename F>
+__device__ __forceinline__ void for_due_records(const KArgs& k,
+                                                const rec_stage& S, int lane,
+                                                uint32_t s, uint64_t n,
+                                                F&& put)
+{
+    const uint32_t r = (uint32_t)lane & (REC_LANES - 1u);
+    const uint32_t row = S.row[s][r];
+    const uint64_t base = S.base[r], row_bytes = S.row_bytes[r];
+    const uint32_t span = S.span[r], what = S.what[r];
+    const uint32_t nrec = lane_u32(S.nrec, 0);
+    const uint64_t dst = base + row_bytes * row;
+    unsigned long long todo = __ballot((uint32_t)lane < REC_LANES &&
+                                       (uint32_t)lane < nrec &&
+                                       row != REC_NOT);
+    while (todo != 0ull) {
+        const int i = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const uint32_t sp = lane_u32(span, i), w = lane_u32(what, i);
+        put(reinterpret_cast<double*>(lane_u64(dst, i)),
+            (int32_t)(sp & 0xffffu), (int32_t)(sp >> 16), w & 0xffu, w >> 8);
+    }
+    for (uint32_t i = REC_LANES; i < nrec; i++) {
+        const dev_record R = scalar_record(k, lane_u32(S.r_lo, 0) + i);
+        if (record_skipped(R) || !record_now(R.ratio, R.rows, n)) {
+            continue;
+        }
+        const int64_t tile0 = (int64_t)lane_u64((uint64_t)S.tile0, 0);
+        const uint32_t sp = record_span(
+            R, tile0, (int64_t)lane_u64((uint64_t)S.own_lo, 0),
+            (int64_t)lane_u64((uint64_t)S.own_hi, 0));
+        put(reinterpret_cast<double*>(record_base(
+                R, (uint64_t)floor(R.ratio * (double)n), tile0)),
+            (int32_t)(sp & 0xffffu), (int32_t)(sp >> 16), R.type, R.row_idx);
     }
 }
 
@@ -236,9 +398,91 @@ __device__ __forceinline__ void add_shift(const KArgs& k, int32_t m,
     }
 }
 
-/* sources staged per launch in LDS (values for the block's steps) */
-constexpr int TILE_SOURCES = 8;
-constexpr int MAX_BLOCK = 64; /* largest temporal block */
+constexpr uint32_t TILE_SOURCES = 8; /* of a tile, staged in LDS */
+constexpr int MAX_BLOCK = 64;   /* largest temporal block */
+
+/* Source values of a tile for the steps of the block: the first one's in a
+ * register, one step per lane (REG: read by readlane; an LDS read in the
+ * step's chain cost 165 of 410 cycles of the two-level Bloch step), the first
+ * TILE_SOURCES otherwise in LDS, any more from memory.  where: offset of the source's
+ * cell in the tile (the tile's first cell, halo included, has offset 0) and,
+ * in bit 0, its type. */
+__device__ __forceinline__ uint32_t source_where(const KArgs& k, uint32_t i,
+                                                 int64_t tile0)
+{
+    return ((uint32_t)((int64_t)as_const(k.src)[i].gx - tile0) << 1) |
+        (as_const(k.src)[i].type == MBH_SRC_HARD ? 1u : 0u);
+}
+struct tile_sources {
+    uint32_t lo, count;
+    uint32_t where0;
+    double v0;
+};
+__device__ __forceinline__ double source_load(const KArgs& k, uint32_t i,
+                                              uint64_t n, bool in)
+{
+    /* (a run's last value where the step lies beyond the block) */
+    return k.src_data[(uint64_t)i * k.n_t + (in ? n : 0u)];
+}
+template<bool REG>
+__device__ __forceinline__ tile_sources stage_sources(
+    const KArgs& k, double (*S)[MAX_BLOCK], int lane, bool writer,
+    const tile_meta& M, int64_t tile0, uint64_t n0, uint32_t nsteps)
+{
+    tile_sources T{ M.src_lo, M.src_hi - M.src_lo, 0u, 0.0 };
+    if (T.count > 0) {
+        const bool in = lane < (int)nsteps;
+        const uint64_t n = n0 + (uint64_t)lane;
+        if constexpr (REG) {
+            T.where0 = source_where(k, T.lo, tile0);
+            T.v0 = source_load(k, T.lo, n, in);
+        }
+        if (T.count > (REG ? 1u : 0u)) {
+            if (writer) {
+                const uint32_t cnt =
+                    T.count < TILE_SOURCES ? T.count : TILE_SOURCES;
+                for (uint32_t j = REG ? 1u : 0u; j < cnt; j++) {
+                    S[j][lane] = source_load(k, T.lo + j, n, in);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    return T;
+}
+/* calls put(offset, hard, value) for every source of the tile, in list
+ * order (solver_cpu_fdtd.tpp:247-255) */
+template<bool REG, typename F>
+__device__ __forceinline__ void for_sources(const KArgs& k,
+                                            const double (*S)[MAX_BLOCK],
+                                            const tile_sources& T,
+                                            int64_t tile0, uint64_t n0,
+                                            uint32_t s, F&& put)
+{
+    if (T.count == 0) {
+        return;
+    }
+    if constexpr (REG) {
+        put((int32_t)(T.where0 >> 1), (T.where0 & 1u) != 0u,
+            lane_f64(T.v0, (int)s));
+    }
+    for (uint32_t j = REG ? 1u : 0u; j < T.count; j++) {
+        const uint32_t w = source_where(k, T.lo + j, tile0);
+        double v;
+        if (j < TILE_SOURCES) {
+            v = S[j][s];
+        } else {
+            v = as_const(k.src_data)[(uint64_t)(T.lo + j) * k.n_t + n0 + s];
+        }
+        put((int32_t)(w >> 1), (w & 1u) != 0u, v);
+    }
+}
+
+/* LDS of a tile: the sources' values for the block's steps, the records */
+struct tile_lds {
+    double src[TILE_SOURCES][MAX_BLOCK];
+    rec_stage rec;
+};
 
 /* One tile t: all steps of the temporal block for the tile's cells.
  * With W > 1 the tile spans W wavefronts of one workgroup, each holding a
@@ -247,12 +491,12 @@ constexpr int MAX_BLOCK = 64; /* largest temporal block */
  * update) come through LDS every step, so only the tile's two outer edges
  * carry a halo (64 C W - 2 tb owned cells instead of 64 C - 2 tb). */
 template<class A, int C, typename ST, bool RED = false, int W = 1>
-__device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
+__device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
+                                          tile_lds& lds)
 {
     static_assert(W == 1 || !RED, "multi-wavefront tiles: plain order only");
     static_assert(W == 1 || A::STAGE == 0,
                   "multi-wavefront tiles: no per-wavefront LDS staging");
-    __shared__ double s_src[TILE_SOURCES][MAX_BLOCK];
     /* boundary values of each wavefront's run for its neighbours */
     __shared__ double x_h[W > 1 ? W : 1]; /* H of the first cell */
     __shared__ double x_e[W > 1 ? W : 1]; /* E of the last cell */
@@ -265,13 +509,19 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
                                                          : (int64_t)k.Gown;
     const int64_t gl =
         own_lo - (int64_t)k.halo + (int64_t)(wv * 64 + lane) * C;
+    const int64_t tile0 = own_lo - (int64_t)k.halo;
     const uint64_t n0 = *as_const(k.n_base) + k.n_off;
     const uint32_t nsteps = k.nsteps;
+    const tile_meta M{ as_const(k.tiles)[t].src_lo,
+                       as_const(k.tiles)[t].src_hi,
+                       as_const(k.tiles)[t].rec_lo,
+                       as_const(k.tiles)[t].rec_hi };
 
     double e[C], h[C], p[C];
     double fa[C], fb[C], fc[C], fg[C], fx[C];
     typename A::state d[C];
-    int32_t m[C];
+    int32_t m[C];  /* material (-1: outside the grid) */
+    int32_t ma[C]; /* the same where it has a density, else -1 */
     bool hz[C];
 
     /* The state loads of all cells first, each from a clamped address
@@ -293,7 +543,9 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
         for (int j = 0; j < A::DC; j++) {
             dv[j] = ld<ST>(k.d_in, (uint64_t)j * k.dstride + gc);
         }
-        m[c] = in ? mv : -1;
+        m[c] = in ? mat_of(mv) : -1;
+        ma[c] = (A::DC > 0 && in && mv >= 0 && (mv & MAT_QM) != 0) ? m[c]
+                                                                   : -1;
         hz[c] = in ? (hv != 0) : true;
         e[c] = in ? ev : 0.0;
         /* the trailing pseudo cell is never owned, so never written back:
@@ -308,6 +560,16 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
             d[c].v[j] = in ? dv[j] : 0.0;
         }
     }
+    /* the tile's records, one per lane, and its sources (the larger z-forms
+     * have no register pair to spare) */
+    constexpr bool SRC_REG = A::DC < 24;
+    dev_record rec_own{};
+    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
+        rec_own = k.tile_rec[M.rec_lo + lane];
+    }
+    const tile_sources srcs =
+        stage_sources<SRC_REG>(k, lds.src, lane, wv == 0, M, tile0, n0,
+                               nsteps);
 #pragma unroll
     for (int c = 0; c < C; c++) {
         if constexpr (A::SHIFT && std::is_same<ST, float>::value) {
@@ -344,19 +606,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
      * the medium); the other lanes of the tile (a cell of another density
      * material, or one lane straddling the interface) take one update per
      * material. The arithmetic of a cell is the same either way. */
-    int32_t ma[C];
     int32_t first = -1;
-#pragma unroll
-    for (int c = 0; c < C; c++) {
-        bool act = false;
-        if constexpr (A::DC > 0) {
-            /* material 0's flag read where the cell has none */
-            const bool q = A::has_qm(
-                (cdp)k.qm + (uint64_t)(m[c] < 0 ? 0 : m[c]) * k.qstride);
-            act = (m[c] >= 0) && q;
-        }
-        ma[c] = act ? m[c] : -1;
-    }
 #pragma unroll
     for (int c = C - 1; c >= 0; c--) {
         first = (ma[c] >= 0) ? ma[c] : first;
@@ -375,7 +625,8 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
     cdp q0 = (cdp)k.qm + (uint64_t)(m1 < 0 ? 0 : m1) * k.qstride;
     const bool q0_active = m1 >= 0;
     /* doubles of the material blob the algorithm wants staged in LDS */
-    constexpr int STAGE = A::STAGE;
+    constexpr bool ROWS = A::ROWC && C == 1;
+    constexpr int STAGE = ROWS ? 0 : A::STAGE;
     __shared__ double s_q[STAGE > 0 ? STAGE : 1];
     if constexpr (STAGE > 0) {
         if (q0_active) {
@@ -386,20 +637,6 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
         __syncthreads();
     }
 
-    /* sources of this tile: their values for the block's steps go to LDS */
-    const uint32_t s_lo = as_const(k.tile_src)[2 * t];
-    const uint32_t s_hi = as_const(k.tile_src)[2 * t + 1];
-    const uint32_t nsrc = s_hi - s_lo;
-    const bool src_staged = nsrc <= TILE_SOURCES && nsteps <= MAX_BLOCK;
-    if (src_staged && nsrc > 0) {
-        if (wv == 0) {
-            for (uint32_t j = 0; j < nsrc; j++) {
-                const double* data = as_const(k.src)[s_lo + j].data;
-                s_src[j][lane] = (lane < (int)nsteps) ? data[n0 + lane] : 0.0;
-            }
-        }
-        __syncthreads();
-    }
     if constexpr (W > 1) {
         if (lane == 0) {
             x_h[wv] = h[0];
@@ -408,23 +645,92 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
     }
 
     /* steps of this block at which any of the tile's records is due */
-    const uint32_t r_lo = as_const(k.tile_rec_ptr)[t];
-    const uint32_t r_hi = as_const(k.tile_rec_ptr)[t + 1];
-    uint64_t rec_steps = 0;
-    for (uint32_t ri = r_lo; ri < r_hi; ri++) {
-        const uint32_t idx = as_const(k.tile_rec_idx)[ri];
-        const double ratio = as_const(k.rec)[idx].ratio;
-        const uint64_t rows = as_const(k.rec)[idx].rows;
-        rec_steps |= __ballot(lane < (int)nsteps &&
-                              record_now(ratio, rows, n0 + lane));
-    }
+    uint64_t rec_steps = stage_records(k, lds.rec, rec_own, lane, wv == 0, M,
+                                       own_lo, own_hi, n0, nsteps);
+
+    /* material constants held over the steps: each lane's own with one cell
+     * per lane, m1's otherwise */
+    constexpr bool LANE = A::CONSTS && C == 1;
+    auto consts = [&]() {
+        if constexpr (LANE) {
+            const auto q = A::load(
+                (const double*)k.qm +
+                (uint64_t)(ma[0] < 0 ? 0 : ma[0]) * k.qstride);
+            return ma[0] >= 0 ? q : A::one();
+        } else if constexpr (A::CONSTS) {
+            return A::load(q0);
+        } else {
+            return 0;
+        }
+    }();
+
+    /* or m1's, sixteen to a register pair; others: lanes of a tile with a
+     * second density material */
+    auto rows = [&]() {
+        if constexpr (ROWS) {
+            return typename A::rowc();
+        } else {
+            return 0;
+        }
+    }();
+    auto load_rows = [&](int32_t mm) {
+        if constexpr (ROWS) {
+            const uint64_t at = (uint64_t)(mm < 0 ? 0 : mm) * k.qstride;
+            rows.load((cdp)k.qm + at, (const double*)k.qm + at);
+        }
+    };
+    load_rows(m1);
+    const unsigned long long others =
+        ROWS ? __ballot(ma[0] >= 0 && ma[0] != m1) : 0ull;
 
     /* density update of every cell from its current field
      * (solver_cpu_fdtd.tpp:278-285, solver_cpu_fdtd_red.tpp:451-457) */
     auto density_update = [&]() {
-        if constexpr (A::DC > 0) {
+        if constexpr (LANE) {
+            A::template apply<1>(consts, d, e, p);
+        } else if constexpr (ROWS) {
+            if (m1 >= 0) {
+                /* Every lane computes with the constants of one material
+                 * (the row registers need all lanes active), that
+                 * material's cells keep the result; tiles with a second
+                 * density material repeat it with that one's constants. */
+                unsigned long long left = others;
+                typename A::state old;
+                double pold = 0.0;
+                for (int32_t mm = m1;;) {
+                    const bool mine = full1 || ma[0] == mm;
+                    if (!full1) {
+                        old = d[0];
+                        pold = p[0];
+                    }
+                    A::apply_rows(rows, d[0], e[0], p[0], mine);
+                    if (full1) {
+                        break;
+                    }
+#pragma unroll
+                    for (int j = 0; j < A::DC; j++) {
+                        d[0].v[j] = mine ? d[0].v[j] : old.v[j];
+                    }
+                    p[0] = mine ? p[0] : pold;
+                    if (others == 0ull) {
+                        break;
+                    }
+                    mm = left != 0ull
+                        ? __builtin_amdgcn_readlane(ma[0],
+                                                    __builtin_ctzll(left))
+                        : m1;
+                    load_rows(mm);
+                    if (left == 0ull) {
+                        break;
+                    }
+                    left &= ~__ballot(ma[0] == mm);
+                }
+            }
+        } else if constexpr (A::DC > 0) {
             auto update_m1 = [&]() {
-                if constexpr (STAGE > 0) {
+                if constexpr (A::CONSTS) {
+                    A::template apply<C>(consts, d, e, p);
+                } else if constexpr (STAGE > 0) {
                     /* an offset the compiler cannot see through keeps the
                      * LDS reads inside the step (hoisted, the staged
                      * constants would occupy VGPRs for the whole loop) */
@@ -460,9 +766,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
         }
     };
 
-    for (uint32_t s = 0; s < nsteps; s++) {
-        const uint64_t n = n0 + s;
-
+    auto step = [&](uint32_t s) __attribute__((always_inline)) {
         if constexpr (RED) {
             density_update();
         }
@@ -496,22 +800,19 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
         }
 
         /* sources, in list order (solver_cpu_fdtd.tpp:247-255) */
-        if (nsrc > 0) {
-            for (uint32_t j = 0; j < nsrc; j++) {
-                const uint64_t gx = as_const(k.src)[s_lo + j].gx;
-                const uint32_t type = as_const(k.src)[s_lo + j].type;
-                const double v = src_staged
-                    ? s_src[j][s]
-                    : as_const(k.src)[s_lo + j].data[n];
-                const int64_t off = (int64_t)gx - gl;
+        for_sources<SRC_REG>(k, lds.src, srcs, tile0, n0, s,
+                    [&](int32_t at, bool hard, double v)
+                        __attribute__((always_inline)) {
+                        const int32_t off =
+                            at - (int32_t)(wv * 64 + lane) * C;
 #pragma unroll
-                for (int c = 0; c < C; c++) {
-                    if (off == c) {
-                        en[c] = (type == MBH_SRC_HARD) ? v : en[c] + v;
-                    }
-                }
-            }
-        }
+                        for (int c = 0; c < C; c++) {
+                            /* (selects: as branches the compiler makes an
+                             * indexed store of them, en in scratch) */
+                            const double x = hard ? v : en[c] + v;
+                            en[c] = off == c ? x : en[c];
+                        }
+                    });
 
         /* H update and boundary condition (solver_cpu_fdtd.tpp:263-275) */
         double e_left = from_left(en[C - 1]);
@@ -552,30 +853,66 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
         if constexpr (!RED) {
             density_update();
         }
-
-        /* record copy (solver_cpu_fdtd.tpp:288-325) */
-        if ((rec_steps >> s) & 1ull) {
-            for (uint32_t ri = r_lo; ri < r_hi; ri++) {
-                const dev_record R =
-                    load_record(k.rec, as_const(k.tile_rec_idx)[ri]);
-                if (!record_now(R.ratio, R.rows, n)) {
-                    continue;
-                }
-                if (R.type == MBH_REC_DENSITY && R.row_idx != R.col_idx) {
-                    continue; /* coherences are not recorded */
-                }
-                const uint64_t row = (uint64_t)floor(R.ratio * (double)n);
+    };
+    /* record copy (solver_cpu_fdtd.tpp:288-325) */
+    auto record = [&](uint32_t s) __attribute__((always_inline)) {
+            for_due_records(
+                k, lds.rec, lane, s, n0 + s,
+                [&](double* dst, int32_t lo, int32_t hi, uint32_t type,
+                    uint32_t row) __attribute__((always_inline)) {
+                    const int32_t o0 = (int32_t)(wv * 64 + lane) * C;
+                    if (type >= MBH_REC_DENSITY) {
+                        /* density, inversion: the constants of one
+                         * material at a time (scalar loads) */
 #pragma unroll
-                for (int c = 0; c < C; c++) {
-                    const int64_t g = gl + c;
-                    if (g >= own_lo && g < own_hi &&
-                        g >= (int64_t)R.gbegin &&
-                        g < (int64_t)(R.gbegin + R.cols)) {
-                        R.dst[row * R.cols + (uint64_t)(g - (int64_t)R.gbegin)] =
-                            record_value<A>(k, R.type, R.row_idx, m[c], e[c],
-                                            h[c], p[c], d[c]);
+                        for (int c = 0; c < C; c++) {
+                            const bool mine = o0 + c >= lo && o0 + c < hi;
+                            for_each_material(
+                                mine ? m[c] : -1, [&](int32_t mm) {
+                                    cdp q = (cdp)k.qm +
+                                        (uint64_t)mm * k.qstride;
+                                    dst[o0 + c] = k.qstride == 0 ? 0.0
+                                        : (type == MBH_REC_INVERSION
+                                               ? A::inversion(q, d[c])
+                                               : A::population(q, d[c],
+                                                               (int)row));
+                                });
+                        }
+                        return;
                     }
-                }
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        if (o0 + c >= lo && o0 + c < hi) {
+                            dst[o0 + c] = type == MBH_REC_ELECTRIC
+                                ? e[c]
+                                : (type == MBH_REC_MAGNETIC ? h[c] : p[c]);
+                        }
+                    }
+                });
+    };
+    if constexpr (A::CONSTS || (A::DC == 0 && A::FAST_FDTD)) {
+        /* short steps: those up to the next one with a due record in a loop
+         * of their own, without a test for records in it (two-level Bloch
+         * form, one cell per lane: 0.305 -> 0.270 us per step; with material
+         * constants read inside the step the nest costs more, 1.35 -> 1.45
+         * us for the reference-order Cayley step) */
+        for (uint32_t s = 0; s < nsteps;) {
+            const uint32_t end = rec_steps != 0ull
+                ? (uint32_t)__builtin_ctzll(rec_steps) + 1u
+                : nsteps;
+            for (; s < end; s++) {
+                step(s);
+            }
+            if (rec_steps != 0ull) {
+                record(s - 1u);
+                rec_steps &= rec_steps - 1ull;
+            }
+        }
+    } else {
+        for (uint32_t s = 0; s < nsteps; s++) {
+            step(s);
+            if ((rec_steps >> s) & 1ull) {
+                record(s);
             }
         }
     }
@@ -612,9 +949,18 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t)
 template<class A, int C>
 constexpr int tile_min_waves()
 {
-    return (std::is_same<A, algo_bloch2r>::value && C == 4)
-        ? MBH_BLOCH2R_WAVES
-        : ((std::is_same<A, algo_bloch2>::value && C == 4) ? 3 : 1);
+    if (std::is_same<A, algo_bloch2r>::value && C == 4) {
+        return MBH_BLOCH2R_WAVES;
+    }
+    if (std::is_same<A, algo_bloch2>::value && C == 4) {
+        return 3;
+    }
+    if (A::DC == 0 && C >= 4) {
+        return C == 4 ? 5 : 3; /* a few registers above the step otherwise */
+    }
+    /* row registers: without a request the polynomial constants of the wide
+     * sin / cos ranges, hoisted out of the steps, fill the file */
+    return A::ROWC && C == 1 ? A::ROWC_WAVES : 1;
 }
 
 template<class A, int C, typename ST, bool RED = false>
@@ -622,8 +968,9 @@ __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(tile_min_waves<A, C>()))) void
 tile_kernel(KArgs k)
 {
-    tile_body<A, C, ST, RED>(k, k.tile_list ? k.tile_list[blockIdx.x]
-                                            : blockIdx.x);
+    __shared__ tile_lds lds;
+    tile_body<A, C, ST, RED>(
+        k, k.tile_list ? k.tile_list[blockIdx.x] : blockIdx.x, lds);
 }
 
 /* tile of W wavefronts (64 W threads) */
@@ -632,8 +979,9 @@ __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(tile_min_waves<A, C>()))) void
 tile_kernel_mw(KArgs k)
 {
-    tile_body<A, C, ST, false, W>(k, k.tile_list ? k.tile_list[blockIdx.x]
-                                                 : blockIdx.x);
+    __shared__ tile_lds lds;
+    tile_body<A, C, ST, false, W>(
+        k, k.tile_list ? k.tile_list[blockIdx.x] : blockIdx.x, lds);
 }
 
 /* ---- launcher registry ------------------------------------------------- */

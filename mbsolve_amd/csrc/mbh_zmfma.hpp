@@ -1,6 +1,11 @@
 /*
  * Rodrigues z-form tile kernel with the generator product on the matrix
- * cores (gfx950 MFMA), for N = 3..6 levels (K = N^2 - 1 = 8, 15, 24, 35).
+ * cores (gfx950 MFMA), for N = 4..6 levels (K = N^2 - 1 = 15, 24, 35).
+ * (Three levels, K = 8, take the VALU z-form with its constants in row
+ * registers: 112 FP64 instructions per cell and step, where the product's
+ * rotation, FP16 split and accumulation around one 16 x 16 tile took about
+ * 140; 65536 cells 1.23 -> 1.11 us per step, with the FP64 product's
+ * accuracy.)
  *
  * One step of the z-form (lindblad_cvr_rodr::update,
  * algo_lindblad_cvr_rodr.hpp:234-268, restated in the rotated basis):
@@ -8,9 +13,8 @@
  * The affine part and the rotation stay in FP64; the product (W - I) r,
  * a K x K matrix shared by all cells of a material times the K x 64 block
  * of the tile's rotated states, runs as v_mfma_f32_16x16x32_f16 on FP16
- * pieces: A = W - I as hi + lo (or hi + mid + lo with ZM_A_PIECES = 3),
- * r as hi + lo; products A_hi r_hi + A_hi r_lo (+ A_mid r_hi) + A_lo r_hi
- * with FP32 accumulation.  A is scaled by a power of two into the FP16
+ * pieces: A = W - I as hi + lo, r as hi + lo; products A_hi r_hi +
+ * A_hi r_lo + A_lo r_hi with FP32 accumulation.  A is scaled by a power of two into the FP16
  * range; the products are scaled back in the FP64 accumulation.  The
  * relative error of the product is about 2^-22 per step.  The A fragments
  * live in LDS (each lane reads back only its own slots).
@@ -34,10 +38,6 @@
 #include "mbh_tile.hpp"
 
 namespace mbh {
-
-#ifndef ZM_A_PIECES
-#define ZM_A_PIECES 2
-#endif
 
 typedef _Float16 zm_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 zm_h2 __attribute__((ext_vector_type(2)));
@@ -67,11 +67,7 @@ struct zm_geom {
     static constexpr bool CFOLD = (ROWS % 8) != 0;
     /* header: [0] 2^-s (scale of the product) [1] max theta_dt
      *         [2] b (p offset) [3] has_qm */
-    /* FP16 pieces of A = W - I: hi + lo (AP = 2) or hi + mid + lo (3).
-     * Three levels at optical frequencies put the free precession in W - I
-     * (omega dt ~ 5e-3 per step): its representation error would act as a
-     * frequency shift, so it gets three pieces. */
-    static constexpr int AP = (N <= 3) ? 3 : ZM_A_PIECES;
+    static constexpr int AP = 2; /* FP16 pieces of A = W - I: hi + lo */
     static constexpr int NF = MT * KC * AP;  /* A fragments */
     static constexpr uint64_t FRAG = 32;     /* zm_h8 [MT][KC][AP][64] */
     static constexpr uint64_t TH = FRAG + (uint64_t)NF * 64 * 16;
@@ -270,9 +266,8 @@ __device__ __forceinline__ void zm_step(const zm_consts<N>& K_,
                 bl[kc][sl + 1] = lo[1];
             }
         }
-        /* (W - I) r of this block = A_hi r_hi + A_hi r_lo [+ A_mid r_hi]
-         * + A_lo r_hi: W - I to about 2^-22 (two pieces) or 2^-33 (three),
-         * r to about 2^-22 (a rounding that changes from step to step).
+        /* (W - I) r of this block = A_hi r_hi + A_hi r_lo + A_lo r_hi: W - I
+         * and r to about 2^-22 (r's rounding changes from step to step).
          * Issued here, so the next block's VALU work overlaps them. */
 #pragma unroll
         for (int t = 0; t < Gm::MT; t++) {
@@ -284,10 +279,6 @@ __device__ __forceinline__ void zm_step(const zm_consts<N>& K_,
                                                            0, 0, 0);
                 a = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bl[kc], a,
                                                            0, 0, 0);
-                if constexpr (Gm::AP == 3) {
-                    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                        af[f + 1], bh[kc], a, 0, 0, 0);
-                }
                 a = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     af[f + Gm::AP - 1], bh[kc], a, 0, 0, 0);
             }
@@ -310,25 +301,22 @@ __device__ __forceinline__ void zm_step(const zm_consts<N>& K_,
     }
 }
 
-/* Wavefronts per SIMD the compiler is asked to fit: two for N = 3 (165
- * registers instead of 212 unasked; 2 % faster on 65536 cells when
- * measured against the unasked build); none for N >= 4
- * (asked for two, four levels fit in 211 registers but ran 30 % slower;
- * five and six levels would spill).  ZM_WAVES_PER_EU (build option)
+/* Wavefronts per SIMD the compiler is asked to fit: two for N = 4, none
+ * beyond (five and six levels would spill).  ZM_WAVES_PER_EU (build option)
  * overrides it for every N. */
 #ifdef ZM_WAVES_PER_EU
 #define ZM_OCCUPANCY \
     __attribute__((amdgpu_waves_per_eu(ZM_WAVES_PER_EU, ZM_WAVES_PER_EU)))
 #else
 #define ZM_OCCUPANCY \
-    __attribute__((amdgpu_waves_per_eu((N <= 3) ? 2 : 1)))
+    __attribute__((amdgpu_waves_per_eu(N == 4 ? 2 : 1)))
 #endif
 
 template<int N, typename ST>
 __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
 {
     using Gm = zm_geom<N>;
-    __shared__ double s_src[TILE_SOURCES][MAX_BLOCK];
+    __shared__ tile_lds lds;
 
     const int lane = threadIdx.x;
     const int q = lane >> 4, j = lane & 15;
@@ -341,7 +329,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
      * materials, and the constant loads start at once. */
     if (!k.tile_mat || blockIdx.x < k.n_mixed) {
         /* (without the table every tile takes the VALU body) */
-        tile_body<algo_zform<N>, 1, ST>(k, t);
+        tile_body<algo_zform<N>, 1, ST>(k, t, lds);
         return;
     }
     const int32_t tm = as_const(k.tile_mat)[blockIdx.x];
@@ -353,12 +341,20 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
     const int64_t gl = g0 + lane;
     const uint64_t n0 = *as_const(k.n_base) + k.n_off;
     const uint32_t nsteps = k.nsteps;
+    const tile_meta M{ as_const(k.tiles)[t].src_lo,
+                       as_const(k.tiles)[t].src_hi,
+                       as_const(k.tiles)[t].rec_lo,
+                       as_const(k.tiles)[t].rec_hi };
+    dev_record rec_own{};
+    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
+        rec_own = k.tile_rec[M.rec_lo + lane];
+    }
 
     /* FDTD state, one cell per lane (folded constants as in tile_kernel) */
     const bool in = (gl >= 0) && (gl < (int64_t)k.G);
     /* a uniform tile lies inside the grid: every lane has the material
      * (the loads go to a clamped address, without a branch of their own) */
-    const int32_t m = tm & ~TILE_MAT_QM;
+    const int32_t m = tm & ~MAT_QM;
     const uint64_t glc = in ? (uint64_t)gl : 0u;
     const uint8_t hzv = k.hzero[glc];
     const double e0 = ld<ST>(k.e_in, glc);
@@ -402,7 +398,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
     /* material constants of the tile (one material, from the table) */
     const int32_t m0 = m;
     const char* fbase = static_cast<const char*>(k.frag);
-    const bool q0_active = (tm & TILE_MAT_QM) != 0;
+    const bool q0_active = (tm & MAT_QM) != 0;
     /* FP32 storage holds y - y* (y* = -Q^T d_in, the relaxation
      * equilibrium, at OFF_YEQ of the material's z-form blob): the stored
      * value and its rounding scale with the distance from equilibrium */
@@ -435,34 +431,11 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
     }
     const bool my_qm = q0_active; /* this lane's cell has a density */
 
-    /* sources of this tile */
-    const uint32_t s_lo = as_const(k.tile_src)[2 * t];
-    const uint32_t s_hi = as_const(k.tile_src)[2 * t + 1];
-    const uint32_t nsrc = s_hi - s_lo;
-    const bool src_staged = nsrc <= TILE_SOURCES && nsteps <= MAX_BLOCK;
-    if (src_staged && nsrc > 0) {
-        for (uint32_t jj = 0; jj < nsrc; jj++) {
-            const double* data = as_const(k.src)[s_lo + jj].data;
-            s_src[jj][lane] = (lane < (int)nsteps) ? data[n0 + lane] : 0.0;
-        }
-        __syncthreads();
-    }
-
-    /* record steps of this block */
-    const uint32_t r_lo = as_const(k.tile_rec_ptr)[t];
-    const uint32_t r_hi = as_const(k.tile_rec_ptr)[t + 1];
-    uint64_t rec_steps = 0;
-    bool rec_density = false;
-    for (uint32_t ri = r_lo; ri < r_hi; ri++) {
-        const uint32_t idx = as_const(k.tile_rec_idx)[ri];
-        const double ratio = as_const(k.rec)[idx].ratio;
-        const uint64_t rows = as_const(k.rec)[idx].rows;
-        const uint32_t type = as_const(k.rec)[idx].type;
-        rec_steps |= __ballot(lane < (int)nsteps &&
-                              record_now(ratio, rows, n0 + lane));
-        rec_density = rec_density || type == MBH_REC_DENSITY ||
-            type == MBH_REC_INVERSION;
-    }
+    /* sources and records of this tile */
+    const tile_sources srcs =
+        stage_sources<(N < 5)>(k, lds.src, lane, true, M, g0, n0, nsteps);
+    const uint64_t rec_steps = stage_records(
+        k, lds.rec, rec_own, lane, true, M, own_lo, own_hi, n0, nsteps);
 
     /* One step in three parts.  The field part (E update, sources, H
      * update and boundary condition, the field's broadcast to the MFMA
@@ -480,23 +453,17 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
     constexpr bool ZM_TIER0_LOOP = (N >= 6);
     double eb[Gm::NB];
     auto field_step = [&](uint32_t s) __attribute__((always_inline)) -> int {
-        const uint64_t n = n0 + s;
         /* E update */
         const double h_right = from_right(h);
         double en = fma(fx, h_right - h, fma(fg, p, fa * e));
         /* sources, in list order */
-        if (nsrc > 0) {
-            for (uint32_t jj = 0; jj < nsrc; jj++) {
-                const uint64_t gx = as_const(k.src)[s_lo + jj].gx;
-                const uint32_t type = as_const(k.src)[s_lo + jj].type;
-                const double v = src_staged
-                    ? s_src[jj][s]
-                    : as_const(k.src)[s_lo + jj].data[n];
-                if ((int64_t)gx == gl) {
-                    en = (type == MBH_SRC_HARD) ? v : en + v;
-                }
-            }
-        }
+        for_sources<(N < 5)>(k, lds.src, srcs, g0, n0, s,
+                    [&](int32_t at, bool hard, double v)
+                        __attribute__((always_inline)) {
+                        if (at == lane) {
+                            en = hard ? v : en + v;
+                        }
+                    });
         /* H update and boundary condition */
         const double e_left = from_left(en);
         h = fma(fc, en - e_left, hm * h);
@@ -544,7 +511,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
             for (int kk = 0; kk < Gm::K; kk++) {
                 dd[kk] = 0.0;
             }
-            if (rec_density) {
+            if (lane_u32(lds.rec.density, 0) != 0u) {
 #pragma unroll 1
                 for (int kk = 0; kk < Gm::NP; kk++) {
                     double part[Gm::NB];
@@ -579,21 +546,15 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
                     }
                 }
             }
-            for (uint32_t ri = r_lo; ri < r_hi; ri++) {
-                const dev_record R =
-                    load_record(k.rec, as_const(k.tile_rec_idx)[ri]);
-                if (!record_now(R.ratio, R.rows, n)) {
-                    continue;
-                }
-                if (R.type == MBH_REC_DENSITY && R.row_idx != R.col_idx) {
-                    continue; /* coherences are not recorded */
-                }
-                const uint64_t row = (uint64_t)floor(R.ratio * (double)n);
-                if (gl >= own_lo && gl < own_hi &&
-                    gl >= (int64_t)R.gbegin &&
-                    gl < (int64_t)(R.gbegin + R.cols)) {
+            for_due_records(
+                k, lds.rec, lane, s, n,
+                [&](double* dst, int32_t lo, int32_t hi, uint32_t type,
+                    uint32_t row) __attribute__((always_inline)) {
+                    if (lane < lo || lane >= hi) {
+                        return;
+                    }
                     double v;
-                    switch (R.type) {
+                    switch (type) {
                     case MBH_REC_ELECTRIC:
                         v = e;
                         break;
@@ -610,13 +571,11 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
                         v = dd[N * (N - 1)];
                         break;
                     default:
-                        v = cv_population<N>(dd, R.row_idx);
+                        v = cv_population<N>(dd, row);
                         break;
                     }
-                    R.dst[row * R.cols + (uint64_t)(gl - (int64_t)R.gbegin)] =
-                        v;
-                }
-            }
+                    dst[lane] = v;
+                });
         }
     };
 

@@ -603,3 +603,68 @@ def test_rodrigues_planes(gpu, levels, order):
         ctx.close()
         _fp64_close(p, got, oracle.OracleRun(p).run(0, 300,
                                                     order=order).scratch)
+
+
+@pytest.mark.parametrize("form,tile,tol", [
+    ("", 64, 0.0), ("", 256, 0.0), ("zform", 64, 1e-11),
+    ("zform", 256, 1e-11), ("zform", 1024, 1e-11)])
+def test_many_sources_and_records_in_one_tile(gpu, form, tile, tol):
+    """Twelve sources (hard and soft, two at one cell) and 28 point records
+    at every step within a few cells: more than a tile keeps in registers
+    and LDS, so the rest comes from memory; against the oracle."""
+    spec = setups.sit_2lvl(num_gridpoints=1500, endtime=0.05e-12,
+                           num_records=4)
+    dx = 150e-6 / 1499
+    spec["sources"] = [
+        {"kind": "gauss", "name": "g%d" % i, "position":
+         (200.5 + 2 * (i // 2 if i < 2 else i)) * dx, "hard": i in (3, 8),
+         "ampl": 1e8 * (i + 1), "freq": 2e14 + 1e13 * i, "phase": 2e-14,
+         "tau": 1e-14} for i in range(12)]
+    spec["records"] += [
+        {"name": "r%d" % i, "type": (0, 1, 2, 4)[i % 4], "row": 1, "col": 1,
+         "interval": 0.0, "position": (205 + i) * dx} for i in range(26)]
+    spec["records"] += [{"name": "d%d%d" % (i, i), "type": 3, "row": i,
+                         "col": i, "interval": 0.0, "position": 210 * dx}
+                        for i in (1, 2)]
+    sol = _solve(spec, form, temporal_block=12, tile_cells=tile)
+    ref = oracle.OracleRun(sol.problem()).run().records()
+    for r, b in zip(sol.get_results(), ref):
+        a = r.get_data_real()
+        assert np.max(np.abs(b)) > 0.0, r.get_name()
+        if tol == 0.0:
+            assert np.array_equal(a, b), r.get_name()
+        else:
+            assert rel_err(a, b) <= tol, (r.get_name(), rel_err(a, b))
+
+
+@pytest.mark.parametrize("levels,form,tol", [
+    (3, "", 1e-12), (3, "zform", 1e-10), (3, "mfma64", 1e-10),
+    (4, "zform", 1e-10), (4, "mfma64", 1e-6), (6, "zform", 1e-10)])
+def test_two_density_media_in_one_tile(gpu, levels, form, tol):
+    """Two Rodrigues media side by side and a vacuum gap: the tiles at their
+    interfaces update each medium with its own constants.  Populations on
+    the trace-1 scale, fields relative to their maximum."""
+    spec = setups.marskar2011(levels, num_gridpoints=260, endtime=0.1e-12)
+    qm = dict(spec["materials"]["AR_Marsk"]["qm"])
+    qm["carrier_density"] *= 0.3
+    qm["h_diag"] = [1.2 * x for x in qm["h_diag"]]
+    spec["materials"]["AR_2"] = {"qm": qm, "rel_permittivity": 2.0}
+    spec["regions"] = [("a", "AR_Marsk", 0.0, 3.1e-5),
+                       ("b", "AR_2", 3.1e-5, 5e-5),
+                       ("v", "Vacuum", 5e-5, 5.4e-5),
+                       ("c", "AR_Marsk", 5.4e-5, 1e-4)]
+    spec["endtime"] = 0.3e-12
+    spec["sources"][0].update(tau=20e-15, phase=60e-15, ampl=1e9)
+    iv = spec["endtime"] / 10
+    spec["records"] = [{"name": n, "interval": iv}
+                       for n in ("inv12", "e", "p")]
+    spec["records"] += [{"name": "d%d%d" % (i, i), "type": 3, "row": i,
+                         "col": i, "interval": iv}
+                        for i in range(1, levels + 1)]
+    sol = _solve(spec, form, temporal_block=8)
+    ref = oracle.OracleRun(sol.problem()).run().records()
+    for r, b in zip(sol.get_results(), ref):
+        a = r.get_data_real()
+        err = (float(np.max(np.abs(a - b)))
+               if r.get_name()[0] in "di" else rel_err(a, b))
+        assert err <= tol, (r.get_name(), err)
