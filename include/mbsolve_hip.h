@@ -257,10 +257,11 @@ typedef struct mbh_options {
  * problem admits a specialised one (pure Maxwell with every held H cell
  * starting at zero; two-level Bloch form with a diagonal Hamiltonian, a
  * real off-diagonal dipole and lossless materials, held H starting at
- * zero; FP64 Rodrigues whose C1, C2 are rotation planes).  The first two
- * drop terms that are exact zeros, so the results are the same; the planes
- * give the assembled A2's results to rounding.  This flag is for verifying
- * that. */
+ * zero; two-level FP64 Cayley with a diagonal Hamiltonian and a real
+ * off-diagonal dipole; FP64 Rodrigues whose C1, C2 are rotation planes).  All
+ * but the last drop terms that are exact zeros, so the results are the same;
+ * the planes give the assembled A2's results to rounding.  This flag is for
+ * verifying that. */
 #define MBH_OPT_GENERIC 1u
 
 typedef struct mbh_info {
@@ -290,6 +291,10 @@ typedef struct mbh_info {
  * plane (every material's C1, C2 are rotation planes of orthonormal vector
  * pairs, as the set-up builds them) */
 #define MBH_INFO_RODR_PLANES 4u
+/* mbh_info.flags: two-level Cayley in the reference's operation order without
+ * the operations on exact zeros (diagonal real Hamiltonian, real off-diagonal
+ * dipole in every medium; the same results bit for bit) */
+#define MBH_INFO_CAYLEY_REAL 8u
 
 typedef struct mbh_ctx mbh_ctx;
 

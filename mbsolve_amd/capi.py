@@ -85,6 +85,7 @@ class mbh_info(C.Structure):
 MBH_INFO_HZ_ZERO = 1
 MBH_INFO_BLOCH_REAL = 2
 MBH_INFO_RODR_PLANES = 4
+MBH_INFO_CAYLEY_REAL = 8
 MBH_NOALLOC_SCRATCH_BYTES = 64 << 20
 
 

@@ -349,6 +349,28 @@ void zform_pop(uint32_t levels, const double* zq, double* out)
     }
 }
 
+/* algo_cayley2r applies to a medium: diagonal real Hamiltonian, real and
+ * purely off-diagonal symmetric dipole, and an imaginary part of the
+ * determinant that is zero or far from underflow */
+bool cayley2_real(const double* cq)
+{
+    if (cq[0] == 0.0) {
+        return true;
+    }
+    const double* H = cq + 5;
+    const double* mu = H + 8;
+    for (int i = 0; i < 4; i++) {
+        const bool diag = (i == 0 || i == 3);
+        if (H[2 * i + 1] != 0.0 || mu[2 * i + 1] != 0.0 ||
+            (diag ? mu[2 * i] : H[2 * i]) != 0.0) {
+            return false;
+        }
+    }
+    const double c1 = -(0.5 * (cq[3] * H[6])) - 0.5 * (cq[3] * H[0]);
+    return mu[2] == mu[4] && std::isfinite(c1) &&
+        (c1 == 0.0 || std::fabs(c1) > 1e-100);
+}
+
 uint64_t rodrp_stride(uint32_t levels)
 {
     switch (levels) {
@@ -584,6 +606,7 @@ struct mbh_ctx {
     bool bloch_real = false;
     bool generic = false; /* MBH_OPT_GENERIC: no specialised kernels */
     bool planes = false;  /* FP64 Rodrigues by rotation planes (algo_rodrp) */
+    bool cayley2r = false; /* two-level Cayley media for algo_cayley2r */
     std::vector<int32_t> mat_h; /* per super-grid cell (Bloch conversions) */
     std::vector<double> qm_h;   /* device blob copy (Bloch conversions) */
 
@@ -1098,6 +1121,9 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
     if (ctx->planes) {
         kform = KFORM_RODR_PLANES;
     }
+    if (ctx->cayley2r) {
+        kform = KFORM_CAYLEY2R;
+    }
     ctx->kform = kform;
     std::vector<uint32_t> cs;
     /* cells per lane (tiles of several wavefronts count as their cells
@@ -1438,6 +1464,19 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
     }
     c->generic = (opt.flags & MBH_OPT_GENERIC) != 0;
     const size_t esz = c->fp32 ? sizeof(float) : sizeof(double);
+    /* two-level Cayley in the reference's operation order: without the
+     * operations on exact zeros where every medium allows it */
+    if (c->algo == MBH_ALGO_REG_CAYLEY && c->levels == 2 && !c->bloch &&
+        !c->generic) {
+        c->cayley2r = true;
+        for (uint32_t r = 0; r < num_runs; r++) {
+            for (uint32_t m = 0; m < runs[r].num_materials; m++) {
+                c->cayley2r = c->cayley2r &&
+                    cayley2_real(runs[r].qm_consts +
+                                 (size_t)m * runs[r].qm_stride);
+            }
+        }
+    }
     /* FP64 Rodrigues, three levels and up: by rotation planes where every
      * material's C1, C2 have that form (what the set-up builds); 4 K FMAs
      * per plane instead of 4 K^2 operations */
@@ -2171,6 +2210,9 @@ int mbh_get_info(const mbh_ctx* ctx, mbh_info* info)
     if (ctx->kform == KFORM_BLOCH2R_MIXED ||
         ctx->kform == KFORM_BLOCH2R_ZFORM64) {
         info->flags |= MBH_INFO_BLOCH_REAL;
+    }
+    if (ctx->kform == KFORM_CAYLEY2R) {
+        info->flags |= MBH_INFO_CAYLEY_REAL;
     }
     if (ctx->kform == KFORM_RODR_PLANES) {
         info->flags |= MBH_INFO_RODR_PLANES;

@@ -423,6 +423,162 @@ struct algo_cayley {
 };
 
 /* ======================================================================
+ * algo_cayley<2> for media with a diagonal real Hamiltonian and a real,
+ * purely off-diagonal symmetric dipole (what qm_desc_2lvl builds,
+ * qm_description.hpp:338-432): the same operations in the same order without
+ * those whose operand is an exact zero or one, so the results are bit for
+ * bit those of the general form (up to the sign of zeros).  With
+ * H = diag(a, b) - e u sigma_x, alpha = prop_im a / 2, beta = prop_im b / 2
+ * and gamma = -prop_im e u / 2 the factors are
+ *   I - M/2 = ((1, -alpha), (0, -gamma); (0, -gamma), (1, -beta)),
+ * their determinant is (1 - alpha beta + gamma^2, -alpha - beta), and p needs
+ * the two coherences of rhs only: about 215 FP64 instructions per cell
+ * instead of 430.  The two divisions by |det|^2 share one reciprocal (the
+ * quotients come from the hardware division's own sequence without its
+ * scaling, which is the identity in the range checked here; outside it the
+ * step runs the general update).
+ * ==================================================================== */
+struct algo_cayley2r : algo_cayley<2> {
+    static constexpr bool CONSTS = true;
+    struct consts {
+        double alpha, beta, c0, nc1, c11, hp, u;
+        double D2a, D2b, D1[4], r2a, r2b, a, b, rhs_im, carrier;
+        const double* q; /* the blob (general update) */
+    };
+    template<typename P>
+    __device__ static consts load(P q)
+    {
+        consts k;
+        const double prop_im = q[3];
+        k.rhs_im = q[4];
+        k.carrier = q[1];
+        k.a = q[OFF_H0];
+        k.b = q[OFF_H0 + 6];
+        k.u = q[OFF_MU + 2];
+        k.alpha = 0.5 * (prop_im * k.a);
+        k.beta = 0.5 * (prop_im * k.b);
+        k.c0 = 1.0 - k.alpha * k.beta;
+        const double c1 = -k.beta - k.alpha;
+        k.nc1 = -c1;
+        k.c11 = c1 * c1;
+        k.hp = 0.5 * prop_im;
+        k.D2a = q[OFF_D2 + 1];
+        k.D2b = q[OFF_D2 + 2];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            k.D1[i] = q[OFF_D1 + i];
+        }
+        k.r2a = q[OFF_d2 + 1];
+        k.r2b = q[OFF_d2 + 2];
+        k.q = (const double*)q;
+        return k;
+    }
+    /* a medium without a density: the state stays, p is zero */
+    __device__ static consts one()
+    {
+        consts k{};
+        k.c0 = k.D2a = k.D2b = k.D1[0] = k.D1[3] = 1.0;
+        return k;
+    }
+
+    __device__ static void dissipate2(const consts& k, double* d)
+    {
+        const double* D1 = k.D1;
+        d[2] = k.D2a * d[2];
+        d[3] = k.D2a * d[3];
+        d[4] = k.D2b * d[4];
+        d[5] = k.D2b * d[5];
+        const double r0 = D1[0] * d[0] + D1[1] * d[6];
+        const double i0 = D1[0] * d[1] + D1[1] * d[7];
+        const double r1 = D1[2] * d[0] + D1[3] * d[6];
+        const double i1 = D1[2] * d[1] + D1[3] * d[7];
+        d[0] = r0;
+        d[1] = i0;
+        d[6] = r1;
+        d[7] = i1;
+    }
+
+    template<int C>
+    __device__ static void apply(const consts& k, state* s, const double* e,
+                                 double* p)
+    {
+        double gam[C], dr[C], s2[C];
+        bool ok = true;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            gam[c] = k.hp * (-(e[c] * k.u));
+            dr[c] = k.c0 + gam[c] * gam[c];
+            s2[c] = dr[c] * dr[c] + k.c11;
+            ok = ok && s2[c] >= 0x1p-200 && s2[c] <= 0x1p+200;
+        }
+        if (!__all(ok)) {
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                if (k.q != nullptr) {
+                    algo_cayley<2>::update((cdp)k.q, s[c], e[c], p[c]);
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            double* v = s[c].v;
+            const double g = gam[c], al = k.alpha, be = k.beta;
+            /* 1 / det = (x, y) */
+            double r = __builtin_amdgcn_rcp(s2[c]);
+            double t = fma(-s2[c], r, 1.0);
+            r = fma(r, t, r);
+            t = fma(-s2[c], r, 1.0);
+            r = fma(r, t, r);
+            double x = dr[c] * r;
+            x = fma(fma(-s2[c], x, dr[c]), r, x);
+            double y = k.nc1 * r;
+            y = fma(fma(-s2[c], y, k.nc1), r, y);
+            /* inverse of I - M/2 */
+            const cplx R0{ x + be * y, y - be * x };
+            const cplx R1{ -(g * y), g * x };
+            const cplx R3{ x + al * y, y - al * x };
+            /* U = R (I + M/2) */
+            const double g1r = R1.re * g, g1i = R1.im * g;
+            const cplx U0{ (R0.re - R0.im * al) - g1i,
+                           (R0.re * al + R0.im) + g1r };
+            const cplx U1{ -(R0.im * g) + (R1.re - R1.im * be),
+                           R0.re * g + (R1.re * be + R1.im) };
+            const cplx U2{ (R1.re - R1.im * al) - R3.im * g,
+                           (R1.re * al + R1.im) + R3.re * g };
+            const cplx U3{ -g1i + (R3.re - R3.im * be),
+                           g1r + (R3.re * be + R3.im) };
+            const cplx U[4] = { U0, U1, U2, U3 };
+            dissipate2(k, v);
+            cplx d[4], w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                d[i] = cplx{ v[2 * i], v[2 * i + 1] };
+            }
+            cmatmul<2>(U, d, w);
+            cmatmul_adj<2>(w, U, d);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v[2 * i] = d[i].re;
+                v[2 * i + 1] = d[i].im;
+            }
+            dissipate2(k, v);
+            /* the coherences of rhs = -i/hbar [H0, d] + D(d) */
+            const double q1 =
+                -(k.rhs_im * (k.a * v[3] - v[3] * k.b)) + k.r2a * v[2];
+            const double q2 =
+                -(k.rhs_im * (k.b * v[5] - v[5] * k.a)) + k.r2b * v[4];
+            p[c] = k.carrier * (q1 * k.u + q2 * k.u);
+        }
+    }
+
+    __device__ static void update(cdp q, state& s, double e, double& p)
+    {
+        apply<1>(load(q), &s, &e, &p);
+    }
+};
+
+/* ======================================================================
  * Two-level regularized Cayley in closed Bloch form.  Mathematically the
  * update of algo_cayley<2> (algo_lindblad_reg_cayley.hpp:206-257) for a
  * Hermitian state, rearranged.  With H = h0 I + h.sigma and

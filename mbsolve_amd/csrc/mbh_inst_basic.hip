@@ -2,7 +2,8 @@
  * Kernel instantiations: noop (pure Maxwell) and regularized Cayley.
  * Reference operation order: FP64 storage implements MBH_FORM_FP64, FP32
  * storage MBH_FORM_MIXED (three-level Cayley; noop with the folded FDTD
- * constants).  Two-level Cayley in closed
+ * constants); two-level Cayley also without its exact zeros for a diagonal
+ * Hamiltonian and a real dipole (algo_cayley2r).  Two-level Cayley in closed
  * Bloch form: FP32 storage MBH_FORM_MIXED, FP64 storage MBH_FORM_ZFORM64,
  * each also specialised for a diagonal Hamiltonian and a real dipole
  * (algo_bloch2r, chosen by the host from the constants), the latter also
@@ -33,6 +34,9 @@ template __global__ void tile_kernel<algo_noop_hz0, 8, float>(KArgs);
 template __global__ void tile_kernel<algo_cayley<2>, 1, double>(KArgs);
 template __global__ void tile_kernel<algo_cayley<2>, 2, double>(KArgs);
 template __global__ void tile_kernel<algo_cayley<2>, 4, double>(KArgs);
+template __global__ void tile_kernel<algo_cayley2r, 1, double>(KArgs);
+template __global__ void tile_kernel<algo_cayley2r, 2, double>(KArgs);
+template __global__ void tile_kernel<algo_cayley2r, 4, double>(KArgs);
 template __global__ void tile_kernel<algo_bloch2, 1, float>(KArgs);
 template __global__ void tile_kernel<algo_bloch2, 2, float>(KArgs);
 template __global__ void tile_kernel<algo_bloch2, 4, float>(KArgs);
@@ -78,6 +82,9 @@ const kernel_entry k_table_basic[] = {
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_FP64, 1, algo_cayley<2>, double),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_FP64, 2, algo_cayley<2>, double),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_FP64, 4, algo_cayley<2>, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_CAYLEY2R, 1, algo_cayley2r, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_CAYLEY2R, 2, algo_cayley2r, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_CAYLEY2R, 4, algo_cayley2r, double),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_MIXED, 1, algo_bloch2, float),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_MIXED, 2, algo_bloch2, float),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, MBH_FORM_MIXED, 4, algo_bloch2, float),

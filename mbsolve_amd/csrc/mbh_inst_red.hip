@@ -22,6 +22,8 @@ template __global__ void tile_kernel<algo_noop, 2, double, true>(KArgs);
 template __global__ void tile_kernel<algo_noop, 4, double, true>(KArgs);
 template __global__ void tile_kernel<algo_cayley<2>, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_cayley<2>, 2, double, true>(KArgs);
+template __global__ void tile_kernel<algo_cayley2r, 1, double, true>(KArgs);
+template __global__ void tile_kernel<algo_cayley2r, 2, double, true>(KArgs);
 template __global__ void tile_kernel<algo_cayley<3>, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_cayley<4>, 1, double, true>(KArgs);
 template __global__ void tile_kernel<algo_cayley<5>, 1, double, true>(KArgs);
@@ -46,6 +48,12 @@ const kernel_entry k_table_red[] = {
     MBH_RED_ENTRY(MBH_ALGO_NOOP, 0, 4, algo_noop),
     MBH_RED_ENTRY(MBH_ALGO_REG_CAYLEY, 2, 1, algo_cayley<2>),
     MBH_RED_ENTRY(MBH_ALGO_REG_CAYLEY, 2, 2, algo_cayley<2>),
+    kernel_entry { MBH_ALGO_REG_CAYLEY, 2, KFORM_CAYLEY2R, 1,
+                   &launch_tile<algo_cayley2r, 1, double, true>,
+                   MBH_ORDER_RED },
+    kernel_entry { MBH_ALGO_REG_CAYLEY, 2, KFORM_CAYLEY2R, 2,
+                   &launch_tile<algo_cayley2r, 2, double, true>,
+                   MBH_ORDER_RED },
     MBH_RED_ENTRY(MBH_ALGO_REG_CAYLEY, 3, 1, algo_cayley<3>),
     MBH_RED_ENTRY(MBH_ALGO_REG_CAYLEY, 4, 1, algo_cayley<4>),
     MBH_RED_ENTRY(MBH_ALGO_REG_CAYLEY, 5, 1, algo_cayley<5>),

@@ -113,6 +113,9 @@ constexpr uint32_t KFORM_BLOCH2R_MIXED = 0x101;
 constexpr uint32_t KFORM_BLOCH2R_ZFORM64 = 0x102;
 /* algo_rodrp (FP64 Rodrigues by rotation planes), both step orders */
 constexpr uint32_t KFORM_RODR_PLANES = 0x103;
+/* algo_cayley2r (reference-order two-level Cayley without its exact zeros),
+ * both step orders */
+constexpr uint32_t KFORM_CAYLEY2R = 0x104;
 
 template<typename ST>
 __device__ __forceinline__ double ld(const void* p, uint64_t i)

@@ -605,6 +605,60 @@ def test_rodrigues_planes(gpu, levels, order):
                                                     order=order).scratch)
 
 
+@pytest.mark.parametrize("order", ["plain", "red"])
+@pytest.mark.parametrize("case", ["sit2", "cpml", "huge_field"])
+def test_cayley_without_exact_zeros(gpu, case, order):
+    """Two-level FP64 Cayley for a diagonal Hamiltonian and a real dipole
+    drops only operations on exact zeros and ones: records and state equal
+    those of the general kernel (MBH_OPT_GENERIC) bit for bit, also where the
+    field leaves the range in which the divisions share a reciprocal; a
+    complex dipole takes the general kernel and equals the oracle."""
+    if case == "cpml":
+        spec = setups.tzenov2018_cpml(num_gridpoints=900, endtime=1e-12)
+        iv = spec["endtime"] / 8
+        spec["records"] = [{"name": n, "interval": iv}
+                           for n in ("inv12", "e", "h", "p")]
+    else:
+        spec = setups.sit_2lvl(num_gridpoints=700, endtime=0.15e-12,
+                               num_records=9, phase=1.0)
+        spec["records"].append({"name": "p", "interval":
+                                spec["endtime"] / 8})
+        if case == "huge_field":
+            spec["sources"][0]["ampl"] = 1e29
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, "", order), dev, scen)
+    nt = int(prob["num_timesteps"])
+    out = []
+    for generic, tile in ((True, 64), (False, 64), (False, 128)):
+        print("case cayley", case, order, generic, tile, flush=True)
+        ctx = capi.Context([prob], capi.options(
+            "fp64", temporal_block=8, tile_cells=tile, order=order,
+            generic=generic))
+        assert bool(ctx.info()["flags"] & capi.MBH_INFO_CAYLEY_REAL) == \
+            (not generic)
+        ctx.run(0, nt)
+        out.append((ctx.records(0), ctx.state(0)))
+        ctx.close()
+    assert np.max(np.abs(out[0][0])) > 0 and np.all(np.isfinite(out[0][0]))
+    for rec, st in out[1:]:
+        assert np.array_equal(rec, out[0][0])
+        for k in ("e", "h", "p", "d"):
+            assert np.array_equal(st[k], out[0][1][k]), k
+    other = dict(prob)
+    q = np.array(prob["qm_consts"], dtype=float).reshape(
+        int(prob["num_materials"]), -1)
+    q[:, 5 + 8 + 3] = 0.3 * q[:, 5 + 8 + 2]    # Im mu01 = -Im mu10
+    q[:, 5 + 8 + 5] = -0.3 * q[:, 5 + 8 + 2]
+    other["qm_consts"] = q.ravel()
+    ctx = capi.Context([other], capi.options("fp64", order=order))
+    assert not ctx.info()["flags"] & capi.MBH_INFO_CAYLEY_REAL
+    ctx.run(0, 60)
+    got = ctx.records(0)
+    ctx.close()
+    ref = oracle.OracleRun(other).run(0, 60, order=order).scratch[:len(got)]
+    assert np.array_equal(got, ref)
+
+
 @pytest.mark.parametrize("form,tile,tol", [
     ("", 64, 0.0), ("", 256, 0.0), ("zform", 64, 1e-11),
     ("zform", 256, 1e-11), ("zform", 1024, 1e-11)])
