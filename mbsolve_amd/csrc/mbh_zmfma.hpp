@@ -582,16 +582,23 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
     if constexpr (ZM_TIER0_LOOP) {
         uint32_t s = 0;
         int pending = 0;
-        for (; s < nsteps; s++) {
-            const int tier = field_step(s);
-            if (tier != 0) {
-                pending = tier;
-                break;
+        while (s < nsteps && pending == 0) {
+            const uint64_t left = rec_steps >> s;
+            const uint32_t end = left != 0ull
+                ? s + (uint32_t)__builtin_ctzll(left) + 1u
+                : nsteps;
+            for (; s < end; s++) {
+                pending = field_step(s);
+                if (pending != 0) {
+                    break;
+                }
+                if (q0_active) {
+                    density_step(std::integral_constant<int, 0>());
+                }
             }
-            if (q0_active) {
-                density_step(std::integral_constant<int, 0>());
+            if (pending == 0 && left != 0ull) {
+                record_step(s - 1u);
             }
-            record_step(s);
         }
         if (s < nsteps) {
             /* step s has its field part done and needs a wider tier */
