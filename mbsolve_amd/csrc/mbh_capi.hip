@@ -18,6 +18,7 @@
 
 #include <mutex>
 
+#include "mbh_team.hpp"
 #include "mbh_zmfma.hpp"
 
 using namespace mbh;
@@ -374,15 +375,15 @@ bool cayley2_real(const double* cq)
 uint64_t rodrp_stride(uint32_t levels)
 {
     switch (levels) {
-    case 3: return algo_rodrp<3>::STRIDE;
-    case 4: return algo_rodrp<4>::STRIDE;
-    case 5: return algo_rodrp<5>::STRIDE;
-    case 6: return algo_rodrp<6>::STRIDE;
+    case 3: return team_consts<3>::STRIDE;
+    case 4: return team_consts<4>::STRIDE;
+    case 5: return team_consts<5>::STRIDE;
+    case 6: return team_consts<6>::STRIDE;
     default: return 0;
     }
 }
 
-/* Rotation-plane constants (layout algo_rodrp<N>) of one material from its
+/* Rotation-plane constants (layout algo_rodrp<N>, then team_consts<N>) of one material from its
  * reference blob (MBH_RODR_STRIDE).  Returns false where some plane with a
  * nonzero angle is not C1 = q2 q1^T - q1 q2^T, C2 = -(q1 q1^T + q2 q2^T)
  * with orthonormal q1, q2, to PLANE_TOL per entry (the entries are at most
@@ -466,6 +467,12 @@ bool rodr_planes(uint32_t levels, const double* cq, double* o)
         np++;
     }
     o[1] = (double)np;
+    switch (levels) {
+    case 3: team_consts<3>::fill(o); break;
+    case 4: team_consts<4>::fill(o); break;
+    case 5: team_consts<5>::fill(o); break;
+    case 6: team_consts<6>::fill(o); break;
+    }
     return true;
 }
 
@@ -1108,6 +1115,35 @@ constexpr double FP32_TIE = 0.015;
  * trial launches read the current buffer, write the other one (discarded)
  * and record nothing, so the simulation state is untouched.
  */
+/* Largest number of tiles for the team form of the FP64 Rodrigues kernel.  It
+ * does about the work of the one-wavefront kernel (a little more: E and H and
+ * the LDS exchanges in every wavefront) with all SIMDs of a CU, so it wins
+ * while tiles are few.  us per step, one wavefront / team: three levels 1.48 /
+ * 1.25 on 256 tiles, 1.46 / 1.37 on 308, 1.41 / 1.41 on 512, 2.0 / 2.6 on
+ * 1261; four levels 9.2 / 8.2 on 1261, 13.2 / 15.2 on 2521; five levels 10.9 /
+ * 8.9 on 512, 10.8 / 11.2 on 683, 19.2 / 20.7 on 1261; six levels 26.5 / 18.8
+ * on 683, 54 / 34 on 1261, 141 / 131 on 5042 (always, in the kernel table):
+ * there the one-wavefront kernel's 19 KB of constants outgrow the scalar
+ * cache.  Both give the same bits. */
+uint64_t team_tiles(uint32_t levels)
+{
+    return levels == 3 ? 384 : (levels == 4 ? 1536 : 512);
+}
+
+/* the kernel for the current geometry */
+tile_launch_fn geometry_kernel(const mbh_ctx* ctx, uint32_t kform)
+{
+    if (kform == KFORM_RODR_PLANES && ctx->C == 1 &&
+        ctx->num_tiles <= team_tiles(ctx->levels)) {
+        const kernel_entry* e = find_kernel(ctx->algo, ctx->levels,
+                                            KFORM_RODR_TEAM, 1, ctx->order);
+        if (e) {
+            return e->fn;
+        }
+    }
+    return find_kernel(ctx->algo, ctx->levels, kform, ctx->C, ctx->order)->fn;
+}
+
 int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
 {
     uint32_t kform = kernel_form(ctx->algo, ctx->levels, ctx->form);
@@ -1188,9 +1224,7 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
             break;
         }
         set_geometry(ctx, cd.first, cd.second);
-        ctx->launch =
-            find_kernel(ctx->algo, ctx->levels, kform, cd.first, ctx->order)
-                ->fn;
+        ctx->launch = geometry_kernel(ctx, kform);
         int rc = build_tile_tables(ctx, false);
         if (rc) {
             return rc;
@@ -1249,8 +1283,7 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
     ctx->tuned_candidates = tried;
     ctx->launch_ms_est = best * pick.second;
     set_geometry(ctx, pick.first, pick.second);
-    ctx->launch =
-        find_kernel(ctx->algo, ctx->levels, kform, ctx->C, ctx->order)->fn;
+    ctx->launch = geometry_kernel(ctx, kform);
     return MBH_OK;
 }
 

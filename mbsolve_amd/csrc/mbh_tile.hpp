@@ -116,6 +116,9 @@ constexpr uint32_t KFORM_RODR_PLANES = 0x103;
 /* algo_cayley2r (reference-order two-level Cayley without its exact zeros),
  * both step orders */
 constexpr uint32_t KFORM_CAYLEY2R = 0x104;
+/* algo_rodrp with a cell's rows split over the wavefronts of a workgroup
+ * (team_kernel) */
+constexpr uint32_t KFORM_RODR_TEAM = 0x105;
 
 template<typename ST>
 __device__ __forceinline__ double ld(const void* p, uint64_t i)
@@ -341,12 +344,13 @@ __device__ __forceinline__ uint64_t stage_records(
 
 /* Calls put(dst, lo, hi, type, level) for every record due at step s of the
  * block (step n of the run), all arguments wave-uniform: the cell at tile
- * offset o in [lo, hi) goes to dst[o]. */
-template<typename F>
+ * offset o in [lo, hi) goes to dst[o].  Of W wavefronts with the same cells,
+ * wavefront wv takes every W-th record. */
+template<int W = 1, typename F>
 __device__ __forceinline__ void for_due_records(const KArgs& k,
                                                 const rec_stage& S, int lane,
                                                 uint32_t s, uint64_t n,
-                                                F&& put)
+                                                F&& put, int wv = 0)
 {
     const uint32_t r = (uint32_t)lane & (REC_LANES - 1u);
     const uint32_t row = S.row[s][r];
@@ -356,6 +360,7 @@ __device__ __forceinline__ void for_due_records(const KArgs& k,
     const uint64_t dst = base + row_bytes * row;
     unsigned long long todo = __ballot((uint32_t)lane < REC_LANES &&
                                        (uint32_t)lane < nrec &&
+                                       (W == 1 || lane % W == wv) &&
                                        row != REC_NOT);
     while (todo != 0ull) {
         const int i = __builtin_ctzll(todo);
@@ -366,7 +371,8 @@ __device__ __forceinline__ void for_due_records(const KArgs& k,
     }
     for (uint32_t i = REC_LANES; i < nrec; i++) {
         const dev_record R = scalar_record(k, lane_u32(S.r_lo, 0) + i);
-        if (record_skipped(R) || !record_now(R.ratio, R.rows, n)) {
+        if ((W > 1 && (int)(i % (uint32_t)W) != wv) || record_skipped(R) ||
+            !record_now(R.ratio, R.rows, n)) {
             continue;
         }
         const int64_t tile0 = (int64_t)lane_u64((uint64_t)S.tile0, 0);

@@ -722,3 +722,43 @@ def test_two_density_media_in_one_tile(gpu, levels, form, tol):
         err = (float(np.max(np.abs(a - b)))
                if r.get_name()[0] in "di" else rel_err(a, b))
         assert err <= tol, (r.get_name(), err)
+
+
+@pytest.mark.parametrize("levels,tiles", [(3, 300), (3, 450), (4, 300),
+                                          (4, 1800), (5, 300), (5, 600),
+                                          (6, 300)])
+def test_rodrigues_rows_over_wavefronts(gpu, levels, tiles):
+    """FP64 Rodrigues with a cell's rows split over wavefronts (few tiles) and
+    by one wavefront (many): the same runs on grids to both sides of the
+    limit, two density media and vacuum in a tile, plane angles from the short
+    series to the library functions; the same bits for every run of a grid as
+    on its own, and the oracle's records to the FP64 form's bound."""
+    spec = _planes_spec(levels)
+    qm = dict(spec["materials"]["AR_Marsk"]["qm"])
+    qm["carrier_density"] *= 0.3
+    qm["h_diag"] = [1.2 * x for x in qm["h_diag"]]
+    spec["materials"]["AR_2"] = {"qm": qm, "rel_permittivity": 2.0}
+    spec["regions"][1:2] = [("a", "AR_Marsk", 3e-5, 5.1e-5),
+                            ("b", "AR_2", 5.1e-5, 7e-5)]
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, ""), dev, scen)
+    nt, n = int(prob["num_timesteps"]), int(prob["num_gridpoints"])
+    runs = tiles * 56 // (n + 1)   # 64 - 2 tb owned cells, tb = 4
+    out = []
+    for count in (1, runs):
+        print("case team", levels, tiles, count, flush=True)
+        ctx = capi.Context([prob] * count, capi.options(
+            "fp64", temporal_block=4, tile_cells=64))
+        info = ctx.info()
+        assert info["flags"] & capi.MBH_INFO_RODR_PLANES
+        assert info["num_tiles"] > 0.9 * tiles or count == 1
+        ctx.run(0, nt)
+        out.append([(ctx.records(r), ctx.state(r))
+                    for r in (0, count // 2, count - 1)])
+        ctx.close()
+    rec, st = out[0][0]
+    for r2, s2 in out[1]:
+        assert np.array_equal(r2, rec)
+        for k in ("e", "h", "p", "d"):
+            assert np.array_equal(s2[k], st[k]), k
+    _fp64_close(prob, rec, oracle.OracleRun(prob).run().scratch)
