@@ -341,6 +341,10 @@ int mbh_elapsed_ms(mbh_ctx* ctx, double* ms);
 int mbh_fetch_records(mbh_ctx* ctx, uint32_t run, double* dst,
                       uint64_t count);
 
+/* The `count` doubles from `first` on of run `run`'s record scratch. */
+int mbh_fetch_record_span(mbh_ctx* ctx, uint32_t run, uint64_t first,
+                          double* dst, uint64_t count);
+
 /* Copies run `run`'s current state to host arrays (any may be NULL):
  * e [N_x], h [N_x + 1], p [N_x], d [N_x][density stride]. */
 int mbh_fetch_state(mbh_ctx* ctx, uint32_t run, double* e, double* h,

@@ -29,9 +29,31 @@ uint32_t env_u32(const char* name, uint32_t dflt)
     return (uint32_t)std::strtoul(v, nullptr, 10);
 }
 
+constexpr uint64_t DIRECT_FETCH = 1u << 15; /* doubles per record */
+
 void copy_results(mbh_ctx* ctx, uint32_t run, const fdtd_problem& p)
 {
     if (p.scratch_size == 0) {
+        return;
+    }
+    /* large records straight into their results; a scratch of less in one
+     * fetch (a fetch of its own costs each record some 20 us) */
+    if (p.scratch_size >= DIRECT_FETCH * p.copy_list.size()) {
+        auto fetch = [&](uint64_t first, real* dst, uint64_t count) {
+            check(mbh_fetch_record_span(ctx, run, first, dst, count), ctx,
+                  "mbh_fetch_record_span");
+        };
+        for (const auto& e : p.copy_list) {
+            if (e.size() == 0) {
+                continue;
+            }
+            fetch(e.dev.offset_real, &*e.res->get_data_real_it(0, 0),
+                  e.size());
+            if (e.dev.is_complex) {
+                fetch(e.dev.offset_imag, &*e.res->get_data_imag_it(0, 0),
+                      e.size());
+            }
+        }
         return;
     }
     std::vector<real> scratch(p.scratch_size);

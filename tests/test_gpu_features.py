@@ -762,3 +762,44 @@ def test_rodrigues_rows_over_wavefronts(gpu, levels, tiles):
         for k in ("e", "h", "p", "d"):
             assert np.array_equal(s2[k], st[k]), k
     _fp64_close(prob, rec, oracle.OracleRun(prob).run().scratch)
+
+
+def test_record_fetch_in_spans(gpu):
+    """Records fetched whole, in spans across the fetch's chunks of 2^18
+    values, and into the results, from two threads at once: the same values;
+    spans outside the scratch are refused."""
+    import threading
+    spec = setups.sit_2lvl(num_gridpoints=40000, endtime=0.02e-12,
+                           num_records=15)
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, "zform"), dev, scen)
+    n = int(prob["scratch_size"])
+    assert n > 2 * (1 << 18) + 5
+    ctx = capi.Context([prob], capi.options("zform64", temporal_block=8))
+    ctx.run(0, int(prob["num_timesteps"]))
+    whole = ctx.records(0)
+    fetch = ctx.lib.mbh_fetch_record_span
+    fetch.argtypes = [capi.C.c_void_p, capi.C.c_uint32, capi.C.c_uint64,
+                      capi._dp, capi.C.c_uint64]
+
+    def span(first, count, out):
+        return fetch(ctx.ctx, 0, first, out.ctypes.data_as(capi._dp), count)
+
+    for first, count in ((0, 1), (7, (1 << 17) - 1), (7, 1 << 17),
+                         (3, (1 << 18) + 1), (n - (1 << 19), 1 << 19)):
+        out = np.full(count, np.nan)
+        assert span(first, count, out) == 0
+        assert np.array_equal(out, whole[first:first + count])
+    for first, count in ((n, 1), (1, n), (0, n + 1), (2 ** 64 - 1, 2)):
+        assert span(first, count, np.zeros(4)) != 0
+    outs = [np.full(n, np.nan) for _ in range(2)]
+    ts = [threading.Thread(target=span, args=(0, n, o)) for o in outs]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert all(np.array_equal(o, whole) for o in outs)
+    ctx.close()
+    sol = _solve(spec, "zform", temporal_block=8)
+    for r, b in zip(sol.get_results(), capi.split_records(prob, whole)):
+        assert np.array_equal(r.get_data_real().ravel(), b.ravel())
