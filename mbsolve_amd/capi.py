@@ -28,7 +28,7 @@ FORMS = {"fp64": MBH_FORM_FP64, "mixed": MBH_FORM_MIXED,
 EXPORTED = ["mbh_version", "mbh_device_count", "mbh_default_options",
             "mbh_create", "mbh_run", "mbh_reset", "mbh_synchronize",
             "mbh_elapsed_ms",
-            "mbh_fetch_records", "mbh_fetch_state",
+            "mbh_fetch_records", "mbh_fetch_record_span", "mbh_fetch_state",
             "mbh_fetch_state_noalloc", "mbh_get_info",
             "mbh_destroy", "mbh_last_error"]
 
@@ -121,6 +121,9 @@ def load():
     lib.mbh_elapsed_ms.argtypes = [vp, C.POINTER(C.c_double)]
     lib.mbh_fetch_records.restype = C.c_int
     lib.mbh_fetch_records.argtypes = [vp, C.c_uint32, _dp, C.c_uint64]
+    lib.mbh_fetch_record_span.restype = C.c_int
+    lib.mbh_fetch_record_span.argtypes = [vp, C.c_uint32, C.c_uint64, _dp,
+                                          C.c_uint64]
     lib.mbh_fetch_state.restype = C.c_int
     lib.mbh_fetch_state.argtypes = [vp, C.c_uint32, _dp, _dp, _dp, _dp]
     lib.mbh_fetch_state_noalloc.restype = C.c_int

@@ -129,6 +129,17 @@ def test_capi_exports_every_declared_symbol():
     assert capi.load().mbh_version().decode().startswith("mbsolve-hip")
 
 
+def test_capi_declares_every_prototype():
+    """Every function of the header has its argument types: without them
+    ctypes passes 64-bit counts and offsets as C int."""
+    lib = capi.load()
+    for n in _header_functions():
+        assert getattr(lib, n).argtypes is not None, n
+    span = lib.mbh_fetch_record_span
+    assert [C.sizeof(t) for t in span.argtypes] == [8, 4, 8, 8, 8]
+    assert span.restype is C.c_int
+
+
 def _good_problem():
     spec = setups.sit_2lvl(num_gridpoints=64, endtime=2e-14, num_records=4)
     dev, scen = setups.build(spec)
