@@ -69,6 +69,17 @@ def _pybind_includes():
             "-I" + sysconfig.get_paths()["include"]]
 
 
+def _check_code(lib):
+    """Inline assembly that the compiler's hazard handling leaves out must
+    keep its wait states in the code made (isa_check.py)."""
+    from mbsolve_amd import isa_check
+    try:
+        isa_check.check(lib)
+    except RuntimeError:
+        os.remove(lib)
+        raise
+
+
 def build(verbose=True, jobs=8):
     os.makedirs(BUILD, exist_ok=True)
     log = print if verbose else (lambda *a, **k: None)
@@ -78,6 +89,7 @@ def build(verbose=True, jobs=8):
     hip_lib = os.path.join(PKG, "libmbsolve_hip.so")
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + hip_objs +
          ["-o", hip_lib])
+    _check_code(hip_lib)
     log("built", hip_lib)
     lib = os.path.join(PKG, "libmbsolve.so")
     _run([CXX, "-shared", "-fPIC"] + cpp_objs +

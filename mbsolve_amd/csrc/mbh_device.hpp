@@ -174,8 +174,10 @@ __device__ __forceinline__ void cinverse(const cplx* A, cplx* R)
  * All lanes must be active: an FMA reads the row's other lanes.
  * DPP reads a register no earlier than two wait states after its write.
  * The registers are written by loads before the steps; pin() at the start of
- * a step keeps those states where the compiler copies one (nothing else
- * writes them, and no kernel that uses them spills). */
+ * a step keeps those states where the compiler copies one there.  Elsewhere
+ * only the register allocator could write one (a copy, a spill); the build
+ * refuses a library whose code has such a write in the two wait states before
+ * a read (isa_check.py). */
 template<int NC>
 struct row_consts {
     static constexpr int NR = (NC + 15) / 16;
