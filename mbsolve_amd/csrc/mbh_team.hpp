@@ -186,10 +186,7 @@ __global__ __launch_bounds__(64 * team_waves<N>()) void team_kernel(KArgs k)
     for (int i = 0; i < R; i++) {
         d[i] = in ? d[i] : 0.0;
     }
-    dev_record rec_own{};
-    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
-        rec_own = k.tile_rec[M.rec_lo + lane];
-    }
+    const dev_record rec_own = own_record(k, M, lane);
     const tile_sources srcs = stage_sources<true>(k, lds.src, lane, wv == 0,
                                                   M, tile0, n0, nsteps);
     const double* f = k.fdtd + (uint64_t)(m < 0 ? 0 : m) * FDTD_STRIDE;
@@ -437,7 +434,7 @@ __global__ __launch_bounds__(64 * team_waves<N>()) void team_kernel(KArgs k)
         if ((rec_steps >> s) & 1ull) {
             for_due_records<W>(
                 k, lds.rec, lane, s, n0 + s,
-                [&](double* dst, int32_t lo, int32_t hi, uint32_t type,
+                [&](record_ptr dst, int32_t lo, int32_t hi, uint32_t type,
                     uint32_t row) __attribute__((always_inline)) {
                     if (lane < lo || lane >= hi) {
                         return;

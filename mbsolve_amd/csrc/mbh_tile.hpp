@@ -258,6 +258,10 @@ __device__ __forceinline__ dev_record scalar_record(const KArgs& k,
     return R;
 }
 
+/* (global, not generic: a generic store holds up the next step's LDS reads
+ * until it is done) */
+typedef __attribute__((address_space(1))) double* record_ptr;
+
 /* where record R goes at row `row`, and its span in the tile */
 __device__ __forceinline__ uint64_t record_base(const dev_record& R,
                                                 uint64_t row, int64_t tile0)
@@ -275,10 +279,19 @@ __device__ __forceinline__ uint32_t record_span(const dev_record& R,
     return lo | (hi << 16);
 }
 
-/* R: lane r's record r of the tile (r < REC_LANES, loaded by the caller
- * together with the state).  Returns the steps of the block at which any of
- * the tile's records is due (one bit per step) and, if there are any, stages
- * them. */
+/* lane r's record r of the tile (r < REC_LANES) */
+__device__ __forceinline__ dev_record own_record(const KArgs& k,
+                                                 const tile_meta& M, int lane)
+{
+    dev_record R{};
+    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
+        R = k.tile_rec[M.rec_lo + lane];
+    }
+    return R;
+}
+
+/* R: own_record.  Returns the steps of the block at which any of the tile's
+ * records is due (one bit per step) and, if there are any, stages them. */
 __device__ __forceinline__ uint64_t stage_records(
     const KArgs& k, rec_stage& S, const dev_record& R, int lane, bool writer,
     const tile_meta& M, int64_t own_lo, int64_t own_hi, uint64_t n0,
@@ -353,10 +366,13 @@ __device__ __forceinline__ void for_due_records(const KArgs& k,
                                                 F&& put, int wv = 0)
 {
     const uint32_t r = (uint32_t)lane & (REC_LANES - 1u);
-    const uint32_t row = S.row[s][r];
-    const uint64_t base = S.base[r], row_bytes = S.row_bytes[r];
-    const uint32_t span = S.span[r], what = S.what[r];
-    const uint32_t nrec = lane_u32(S.nrec, 0);
+    uint64_t base = S.base[r], row_bytes = S.row_bytes[r];
+    uint32_t row = S.row[s][r], span = S.span[r], what = S.what[r];
+    uint32_t n_all = S.nrec;
+    /* (all reads ahead of the first use: one LDS latency) */
+    asm volatile("" : "+v"(base), "+v"(row_bytes), "+v"(row), "+v"(span),
+                      "+v"(what), "+v"(n_all));
+    const uint32_t nrec = lane_u32(n_all, 0);
     const uint64_t dst = base + row_bytes * row;
     unsigned long long todo = __ballot((uint32_t)lane < REC_LANES &&
                                        (uint32_t)lane < nrec &&
@@ -366,21 +382,25 @@ __device__ __forceinline__ void for_due_records(const KArgs& k,
         const int i = __builtin_ctzll(todo);
         todo &= todo - 1;
         const uint32_t sp = lane_u32(span, i), w = lane_u32(what, i);
-        put(reinterpret_cast<double*>(lane_u64(dst, i)),
+        put((record_ptr)(lane_u64(dst, i)),
             (int32_t)(sp & 0xffffu), (int32_t)(sp >> 16), w & 0xffu, w >> 8);
     }
     for (uint32_t i = REC_LANES; i < nrec; i++) {
+        /* (the step number's conversions stay in here: hoisted, they would
+         * hold registers over the steps) */
+        asm volatile("" : "+s"(n));
         const dev_record R = scalar_record(k, lane_u32(S.r_lo, 0) + i);
         if ((W > 1 && (int)(i % (uint32_t)W) != wv) || record_skipped(R) ||
             !record_now(R.ratio, R.rows, n)) {
             continue;
         }
+        const uint64_t at =
+            lane_u64((uint64_t)floor(R.ratio * (double)n), 0);
         const int64_t tile0 = (int64_t)lane_u64((uint64_t)S.tile0, 0);
         const uint32_t sp = record_span(
             R, tile0, (int64_t)lane_u64((uint64_t)S.own_lo, 0),
             (int64_t)lane_u64((uint64_t)S.own_hi, 0));
-        put(reinterpret_cast<double*>(record_base(
-                R, (uint64_t)floor(R.ratio * (double)n), tile0)),
+        put((record_ptr)(record_base(R, at, tile0)),
             (int32_t)(sp & 0xffffu), (int32_t)(sp >> 16), R.type, R.row_idx);
     }
 }
@@ -430,7 +450,7 @@ struct tile_sources {
 __device__ __forceinline__ double source_load(const KArgs& k, uint32_t i,
                                               uint64_t n, bool in)
 {
-    /* (a run's last value where the step lies beyond the block) */
+    /* (lanes beyond the block: the source's first value, not used) */
     return k.src_data[(uint64_t)i * k.n_t + (in ? n : 0u)];
 }
 template<bool REG>
@@ -526,6 +546,24 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
                        as_const(k.tiles)[t].rec_lo,
                        as_const(k.tiles)[t].rec_hi };
 
+    /* The tile's records: staged before the state is loaded they cost
+     * registers of their own only; one cell per lane with its constants in
+     * registers (grids bound by the latency of a launch), and the two-level
+     * Cayley form without its zeros (2^20 cells, 9.1 us per step against
+     * 9.3), have the descriptors in flight together with the state.  Staged after the constants, and
+     * with the record code's addresses kept over the steps, the FP64 noop
+     * kernel spilled (2^27 cells, tiles of 512 cells, blocks of 32 steps:
+     * 65 -> 72 us per step) and three-level Cayley fitted one wavefront per
+     * SIMD instead of two (2^18 cells 14.8 -> 17.4 us per step, 14.5 here). */
+    constexpr bool STAGE_LATE = (C == 1 && (A::CONSTS || A::ROWC)) ||
+        std::is_same<A, algo_cayley2r>::value;
+    uint64_t rec_steps = 0; /* steps of this block with a due record */
+    if constexpr (!STAGE_LATE) {
+        rec_steps =
+            stage_records(k, lds.rec, own_record(k, M, lane), lane, wv == 0,
+                          M, own_lo, own_hi, n0, nsteps);
+    }
+
     double e[C], h[C], p[C];
     double fa[C], fb[C], fc[C], fg[C], fx[C];
     typename A::state d[C];
@@ -569,13 +607,16 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
             d[c].v[j] = in ? dv[j] : 0.0;
         }
     }
-    /* the tile's records, one per lane, and its sources (the larger z-forms
-     * have no register pair to spare) */
-    constexpr bool SRC_REG = A::DC < 24;
-    dev_record rec_own{};
-    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
-        rec_own = k.tile_rec[M.rec_lo + lane];
+    if constexpr (STAGE_LATE) {
+        rec_steps =
+            stage_records(k, lds.rec, own_record(k, M, lane), lane, wv == 0,
+                          M, own_lo, own_hi, n0, nsteps);
     }
+    /* the tile's sources, the first in a register; the larger z-forms and
+     * four or more cells per lane with a density (but for the two-level
+     * Bloch form of a real dipole) have no register pair to spare */
+    constexpr bool SRC_REG = A::DC < 24 &&
+        (C < 4 || A::DC == 0 || std::is_same<A, algo_bloch2r>::value);
     const tile_sources srcs =
         stage_sources<SRC_REG>(k, lds.src, lane, wv == 0, M, tile0, n0,
                                nsteps);
@@ -652,10 +693,6 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
         }
         __syncthreads();
     }
-
-    /* steps of this block at which any of the tile's records is due */
-    uint64_t rec_steps = stage_records(k, lds.rec, rec_own, lane, wv == 0, M,
-                                       own_lo, own_hi, n0, nsteps);
 
     /* material constants held over the steps: each lane's own with one cell
      * per lane, m1's otherwise */
@@ -865,11 +902,18 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
     };
     /* record copy (solver_cpu_fdtd.tpp:288-325) */
     auto record = [&](uint32_t s) __attribute__((always_inline)) {
+            /* (a lane index the compiler cannot see through keeps the
+             * addresses that depend on it out of the steps, where there is
+             * no register to spare) */
+            int ln = lane;
+            if constexpr (A::DC > 0 || C >= 4) {
+                asm volatile("" : "+v"(ln));
+            }
             for_due_records(
-                k, lds.rec, lane, s, n0 + s,
-                [&](double* dst, int32_t lo, int32_t hi, uint32_t type,
+                k, lds.rec, ln, s, n0 + s,
+                [&](record_ptr dst, int32_t lo, int32_t hi, uint32_t type,
                     uint32_t row) __attribute__((always_inline)) {
-                    const int32_t o0 = (int32_t)(wv * 64 + lane) * C;
+                    const int32_t o0 = (int32_t)(wv * 64 + ln) * C;
                     if (type >= MBH_REC_DENSITY) {
                         /* density, inversion: the constants of one
                          * material at a time (scalar loads) */
@@ -920,7 +964,9 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
     } else {
         for (uint32_t s = 0; s < nsteps; s++) {
             step(s);
-            if ((rec_steps >> s) & 1ull) {
+            const bool due = ((rec_steps >> s) & 1ull) != 0ull;
+            /* (unlikely: what spills, spills in the record code) */
+            if (A::DC > 0 ? __builtin_expect(due, false) : due) {
                 record(s);
             }
         }
@@ -964,8 +1010,10 @@ constexpr int tile_min_waves()
     if (std::is_same<A, algo_bloch2>::value && C == 4) {
         return 3;
     }
-    if (A::DC == 0 && C >= 4) {
-        return C == 4 ? 5 : 3; /* a few registers above the step otherwise */
+    /* (266 registers unasked; 2^20 cells 21.1 -> 18.0 us per step with
+     * eleven of them spilled outside the step) */
+    if (std::is_same<A, algo_cayley<2>>::value && C == 4) {
+        return 2;
     }
     /* row registers: without a request the polynomial constants of the wide
      * sin / cos ranges, hoisted out of the steps, fill the file */

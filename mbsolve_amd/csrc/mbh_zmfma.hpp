@@ -345,10 +345,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
                        as_const(k.tiles)[t].src_hi,
                        as_const(k.tiles)[t].rec_lo,
                        as_const(k.tiles)[t].rec_hi };
-    dev_record rec_own{};
-    if ((uint32_t)lane < REC_LANES && (uint32_t)lane < M.rec_hi - M.rec_lo) {
-        rec_own = k.tile_rec[M.rec_lo + lane];
-    }
+    const dev_record rec_own = own_record(k, M, lane);
 
     /* FDTD state, one cell per lane (folded constants as in tile_kernel) */
     const bool in = (gl >= 0) && (gl < (int64_t)k.G);
@@ -548,7 +545,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
             }
             for_due_records(
                 k, lds.rec, lane, s, n,
-                [&](double* dst, int32_t lo, int32_t hi, uint32_t type,
+                [&](record_ptr dst, int32_t lo, int32_t hi, uint32_t type,
                     uint32_t row) __attribute__((always_inline)) {
                     if (lane < lo || lane >= hi) {
                         return;

@@ -1,0 +1,33 @@
+"""Registers and scratch of the built kernels whose speed on large grids hangs
+on the wavefronts that fit a SIMD (512 vector registers, in units of eight)."""
+import pytest
+
+from mbsolve_amd import capi, isa_check
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    return isa_check.resources(capi.LIB_PATH)
+
+
+def _tile(algo, cells, storage="d", red=0):
+    return "_ZN3mbh11tile_kernelINS_%sELi%dE%sLb%dEEEvNS_5KArgsE" % (
+        algo, cells, storage, red)
+
+
+NOOP, CAYLEY, BLOCH = "9algo_noop", "11algo_cayleyILi%dEE", \
+    "13algo_bloch2_tILb0EE"
+
+
+@pytest.mark.parametrize("name,waves,scratch", [
+    (_tile(NOOP, 2), 8, 0), (_tile(NOOP, 4), 5, 0), (_tile(NOOP, 8), 3, 0),
+    (_tile(NOOP, 4, red=1), 5, 0),
+    (_tile(CAYLEY % 2, 1), 4, 0), (_tile(CAYLEY % 2, 4), 2, 48),
+    (_tile(CAYLEY % 2, 1, red=1), 4, 0),
+    (_tile(CAYLEY % 3, 1), 2, 0), (_tile(CAYLEY % 3, 1, "f"), 2, 0),
+    (_tile(BLOCH, 4), 3, 36), (_tile(BLOCH, 4, "f"), 3, 36),
+])
+def test_wavefronts_fit(kernels, name, waves, scratch):
+    k = kernels[name]
+    assert 512 // (-(-k["vgpr"] // 8) * 8) >= waves, k
+    assert k["scratch"] <= scratch, k
