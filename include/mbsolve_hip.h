@@ -255,9 +255,9 @@ typedef struct mbh_options {
 
 /* mbh_options.flags: run the general kernels of the form even where the
  * problem admits a specialised one (pure Maxwell with every held H cell
- * starting at zero; two-level Bloch form with a diagonal Hamiltonian, a
- * real off-diagonal dipole and lossless materials, held H starting at
- * zero; two-level FP64 Cayley with a diagonal Hamiltonian and a real
+ * starting at zero; two-level Bloch form with a real Hamiltonian, a real
+ * dipole whose diagonal does not enter p and lossless materials, held H
+ * starting at zero; two-level FP64 Cayley with a diagonal Hamiltonian and a real
  * off-diagonal dipole; FP64 Rodrigues whose C1, C2 are rotation planes).  All
  * but the last drop terms that are exact zeros, so the results are the same;
  * the planes give the assembled A2's results to rounding.  This flag is for
@@ -283,9 +283,9 @@ typedef struct mbh_info {
 /* mbh_info.flags: the pure-Maxwell FP32 kernel without the H factor of
  * the cells held at zero is in use (every such cell starts with H = 0) */
 #define MBH_INFO_HZ_ZERO 1u
-/* mbh_info.flags: the two-level Bloch kernel specialised for a diagonal
- * Hamiltonian, a real off-diagonal dipole and lossless materials, with
- * every held H cell starting at zero, is in use */
+/* mbh_info.flags: a two-level Bloch kernel specialised for a real
+ * Hamiltonian, a real dipole and lossless materials, with every held H cell
+ * starting at zero, is in use */
 #define MBH_INFO_BLOCH_REAL 2u
 /* mbh_info.flags: FP64 Rodrigues (three levels and up) applies A2 plane by
  * plane (every material's C1, C2 are rotation planes of orthonormal vector

@@ -612,9 +612,10 @@ struct mbh_ctx {
     bool zform = false;
     bool bloch = false; /* two-level Cayley in closed Bloch form */
     /* every Bloch material has beta_y = 0, a field-free alpha0, no p
-     * term in tau and m_z, and no loss (with hz_zero, algo_bloch2r
-     * applies) */
-    bool bloch_real = false;
+     * term in tau and m_z, and no loss (with hz_zero, algo_bloch2s
+     * applies); and beta_x = 0 at e = 0, a field-free beta_z and a trace
+     * that is kept (algo_bloch2r) */
+    bool bloch_real = false, bloch_diag = false;
     bool generic = false; /* MBH_OPT_GENERIC: no specialised kernels */
     bool planes = false;  /* FP64 Rodrigues by rotation planes (algo_rodrp) */
     bool cayley2r = false; /* two-level Cayley media for algo_cayley2r */
@@ -1218,7 +1219,9 @@ int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
         kform = KFORM_NOOP_HZ0;
     }
     if (ctx->bloch && ctx->bloch_real && ctx->hz_zero && !ctx->generic) {
-        kform = ctx->fp32 ? KFORM_BLOCH2R_MIXED : KFORM_BLOCH2R_ZFORM64;
+        kform = ctx->bloch_diag
+            ? (ctx->fp32 ? KFORM_BLOCH2R_MIXED : KFORM_BLOCH2R_ZFORM64)
+            : (ctx->fp32 ? KFORM_BLOCH2S_MIXED : KFORM_BLOCH2S_ZFORM64);
     }
     if (ctx->planes) {
         kform = KFORM_RODR_PLANES;
@@ -1665,19 +1668,23 @@ int mbh_create(const mbh_problem* runs, uint32_t num_runs,
     }
 
     if (c->bloch) {
-        /* algo_bloch2r: beta_x at e = 0, d beta_z / d e, beta_y,
-         * d alpha0 / d e and the p coefficients of tau and m_z exactly zero
-         * and the trace kept in every material with a density, and every
-         * material lossless (fac_a exactly 1) */
-        c->bloch_real = true;
+        /* algo_bloch2s: beta_y, d alpha0 / d e and the p coefficients of
+         * tau and m_z exactly zero in every material with a density, and
+         * every material lossless (fac_a exactly 1); algo_bloch2r: also
+         * beta_x at e = 0 and d beta_z / d e, and the trace kept */
+        c->bloch_real = c->bloch_diag = true;
         for (size_t mi = 0; mi + BLOCH2_STRIDE <= qm.size();
              mi += BLOCH2_STRIDE) {
             const double* o = &qm[mi];
-            if (o[0] != 0.0 &&
-                (o[1] != 0.0 || o[2] != 0.0 || o[5] != 0.0 || o[6] != 0.0 ||
-                 o[8] != 0.0 || o[14] != 0.0 || o[17] != 0.0 ||
-                 o[10] != 1.0 || o[11] != 0.0)) {
+            if (o[0] == 0.0) {
+                continue;
+            }
+            if (o[2] != 0.0 || o[5] != 0.0 || o[8] != 0.0 || o[14] != 0.0 ||
+                o[17] != 0.0) {
                 c->bloch_real = false;
+            }
+            if (o[1] != 0.0 || o[6] != 0.0 || o[10] != 1.0 || o[11] != 0.0) {
+                c->bloch_diag = false;
             }
         }
         for (size_t mi = 0; mi < fdtd.size(); mi += FDTD_STRIDE) {
@@ -2314,7 +2321,9 @@ int mbh_get_info(const mbh_ctx* ctx, mbh_info* info)
         info->flags |= MBH_INFO_HZ_ZERO;
     }
     if (ctx->kform == KFORM_BLOCH2R_MIXED ||
-        ctx->kform == KFORM_BLOCH2R_ZFORM64) {
+        ctx->kform == KFORM_BLOCH2R_ZFORM64 ||
+        ctx->kform == KFORM_BLOCH2S_MIXED ||
+        ctx->kform == KFORM_BLOCH2S_ZFORM64) {
         info->flags |= MBH_INFO_BLOCH_REAL;
     }
     if (ctx->kform == KFORM_CAYLEY2R) {

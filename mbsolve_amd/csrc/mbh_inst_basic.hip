@@ -5,9 +5,9 @@
  * constants); two-level Cayley also without its exact zeros for a diagonal
  * Hamiltonian and a real dipole (algo_cayley2r).  Two-level Cayley in closed
  * Bloch form: FP32 storage MBH_FORM_MIXED, FP64 storage MBH_FORM_ZFORM64,
- * each also specialised for a diagonal Hamiltonian and a real dipole
- * (algo_bloch2r, chosen by the host from the constants), the latter also
- * as tiles of 2 and 4 wavefronts at 4 cells per lane.
+ * each also specialised for a real dipole, with a diagonal Hamiltonian
+ * (algo_bloch2r) and without (algo_bloch2s), chosen by the host from the
+ * constants, these also as tiles of 2 and 4 wavefronts at 4 cells per lane.
  */
 #include "mbh_tile.hpp"
 
@@ -55,6 +55,16 @@ template __global__ void tile_kernel<algo_bloch2r, 2, double>(KArgs);
 template __global__ void tile_kernel<algo_bloch2r, 4, double>(KArgs);
 template __global__ void tile_kernel_mw<algo_bloch2r, 4, 2, double>(KArgs);
 template __global__ void tile_kernel_mw<algo_bloch2r, 4, 4, double>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 1, float>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 2, float>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 4, float>(KArgs);
+template __global__ void tile_kernel_mw<algo_bloch2s, 4, 2, float>(KArgs);
+template __global__ void tile_kernel_mw<algo_bloch2s, 4, 4, float>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 1, double>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 2, double>(KArgs);
+template __global__ void tile_kernel<algo_bloch2s, 4, double>(KArgs);
+template __global__ void tile_kernel_mw<algo_bloch2s, 4, 2, double>(KArgs);
+template __global__ void tile_kernel_mw<algo_bloch2s, 4, 4, double>(KArgs);
 template __global__ void tile_kernel<algo_cayley<3>, 1, double>(KArgs);
 template __global__ void tile_kernel<algo_cayley<3>, 1, float>(KArgs);
 template __global__ void tile_kernel<algo_cayley<4>, 1, double>(KArgs);
@@ -103,6 +113,16 @@ const kernel_entry k_table_basic[] = {
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2R_ZFORM64, 4, algo_bloch2r, double),
     MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2R_ZFORM64, 4, 2, algo_bloch2r, double),
     MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2R_ZFORM64, 4, 4, algo_bloch2r, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_MIXED, 1, algo_bloch2s, float),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_MIXED, 2, algo_bloch2s, float),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_MIXED, 4, algo_bloch2s, float),
+    MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_MIXED, 4, 2, algo_bloch2s, float),
+    MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_MIXED, 4, 4, algo_bloch2s, float),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_ZFORM64, 1, algo_bloch2s, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_ZFORM64, 2, algo_bloch2s, double),
+    MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_ZFORM64, 4, algo_bloch2s, double),
+    MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_ZFORM64, 4, 2, algo_bloch2s, double),
+    MBH_ENTRY_MW(MBH_ALGO_REG_CAYLEY, 2, KFORM_BLOCH2S_ZFORM64, 4, 4, algo_bloch2s, double),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 3, MBH_FORM_FP64, 1, algo_cayley<3>, double),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 3, MBH_FORM_MIXED, 1, algo_cayley<3>, float),
     MBH_ENTRY(MBH_ALGO_REG_CAYLEY, 4, MBH_FORM_FP64, 1, algo_cayley<4>, double),

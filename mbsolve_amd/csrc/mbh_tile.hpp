@@ -111,6 +111,13 @@ __host__ __device__ constexpr int32_t mat_of(int32_t v)
 constexpr uint32_t KFORM_NOOP_HZ0 = 0x100;
 constexpr uint32_t KFORM_BLOCH2R_MIXED = 0x101;
 constexpr uint32_t KFORM_BLOCH2R_ZFORM64 = 0x102;
+/* and algo_bloch2s */
+constexpr uint32_t KFORM_BLOCH2S_MIXED = 0x106;
+constexpr uint32_t KFORM_BLOCH2S_ZFORM64 = 0x107;
+/* two-level Bloch kernels for lossless media with H held at zero */
+template<class A>
+constexpr bool bloch_real = std::is_same<A, algo_bloch2r>::value ||
+    std::is_same<A, algo_bloch2s>::value;
 /* algo_rodrp (FP64 Rodrigues by rotation planes), both step orders */
 constexpr uint32_t KFORM_RODR_PLANES = 0x103;
 /* algo_cayley2r (reference-order two-level Cayley without its exact zeros),
@@ -616,7 +623,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
      * four or more cells per lane with a density (but for the two-level
      * Bloch form of a real dipole) have no register pair to spare */
     constexpr bool SRC_REG = A::DC < 24 &&
-        (C < 4 || A::DC == 0 || std::is_same<A, algo_bloch2r>::value);
+        (C < 4 || A::DC == 0 || bloch_real<A>);
     const tile_sources srcs =
         stage_sources<SRC_REG>(k, lds.src, lane, wv == 0, M, tile0, n0,
                                nsteps);
@@ -831,7 +838,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
             const double hn = (c + 1 < C) ? h[(c + 1) % C] : h_right;
             if constexpr (A::FAST_FDTD && A::DC == 0) {
                 en[c] = fma(fx[c], hn - h[c], fa[c] * e[c]); /* p = 0 */
-            } else if constexpr (std::is_same<A, algo_bloch2r>::value) {
+            } else if constexpr (bloch_real<A>) {
                 /* lossless (fa = 1 in the grid; cells outside it and the
                  * pseudo cells hold E = 0 with fg = fx = 0) */
                 en[c] = fma(fx[c], hn - h[c], fma(fg[c], p[c], e[c]));
@@ -874,7 +881,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
         for (int c = 0; c < C; c++) {
             const double ep = (c > 0) ? en[(c + C - 1) % C] : e_left;
             if constexpr (std::is_same<A, algo_noop_hz0>::value ||
-                          std::is_same<A, algo_bloch2r>::value) {
+                          bloch_real<A>) {
                 /* every held cell starts at zero and its fc is zero */
                 h[c] = fma(fc[c], en[c] - ep, h[c]);
             } else if constexpr (A::FAST_FDTD) {
@@ -1004,7 +1011,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
 template<class A, int C>
 constexpr int tile_min_waves()
 {
-    if (std::is_same<A, algo_bloch2r>::value && C == 4) {
+    if (bloch_real<A> && C == 4) {
         return MBH_BLOCH2R_WAVES;
     }
     if (std::is_same<A, algo_bloch2>::value && C == 4) {

@@ -803,3 +803,50 @@ def test_record_fetch_in_spans(gpu):
     sol = _solve(spec, "zform", temporal_block=8)
     for r, b in zip(sol.get_results(), capi.split_records(prob, whole)):
         assert np.array_equal(r.get_data_real().ravel(), b.ravel())
+
+
+@pytest.mark.parametrize("form,tile", [("mixed", 64), ("mixed", 512),
+                                       ("zform64", 64), ("zform64", 128),
+                                       ("zform64", 1024)])
+def test_bloch_real_dipole_and_mixed_hamiltonian(gpu, form, tile):
+    """A lossless two-level medium with a real off-diagonal Hamiltonian entry
+    beside one with a diagonal Hamiltonian takes the Bloch kernel for real
+    dipoles: records and state of the general kernel bit for bit, the
+    oracle's records to the form's bound."""
+    spec = setups.sit_2lvl(num_gridpoints=1500, endtime=0.2e-12,
+                           num_records=10, phase=1.0)
+    spec["records"].append({"name": "p", "interval": spec["endtime"] / 9})
+    mid, m = [x for x in spec["materials"].items() if x[1].get("qm")][0]
+    w = 0.5 * 2e14 * 2 * np.pi * 1.05457266e-34
+    spec["materials"]["mixed"] = {"qm": {
+        "num_levels": 2, "carrier_density": 1e24, "h_diag": [-w, w],
+        "h_off": [0.05 * w], "mu_diag": [0.0, 0.0],
+        "mu_off": [-1.60217733e-19 * 1e-10],
+        "scattering": [[0.0, 1e9], [2e9, 0.0]], "pure_dephasing": [1e10]}}
+    name, _, x0, x1 = spec["regions"][1]
+    xm = x0 + 0.4 * (x1 - x0)
+    spec["regions"][1:2] = [(name, mid, x0, xm), ("mixed", "mixed", xm, x1)]
+    dev, scen = setups.build(spec)
+    suffix = "zform" if form == "zform64" else form
+    prob = mb.build_problem(setups.solver_name(spec, suffix), dev, scen)
+    nt = int(prob["num_timesteps"])
+    out = []
+    for generic in (False, True):
+        print("case real dipole", form, tile, generic, flush=True)
+        ctx = capi.Context([prob], capi.options(
+            form, temporal_block=8, tile_cells=64 if generic else tile,
+            generic=generic))
+        assert bool(ctx.info()["flags"] & capi.MBH_INFO_BLOCH_REAL) == \
+            (not generic)
+        ctx.run(0, nt)
+        out.append((ctx.records(0), ctx.state(0)))
+        ctx.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    for k in ("e", "h", "p", "d"):
+        assert np.array_equal(out[0][1][k], out[1][1][k]), k
+    ref = oracle.OracleRun(prob).run().records()
+    tol = 1e-5 if form == "mixed" else 1e-10
+    for r, a, b in zip(prob["records"],
+                       capi.split_records(prob, out[0][0]), ref):
+        assert np.max(np.abs(b)) > 0.0, r["type"]
+        assert rel_err(a, b) <= tol, (r["type"], rel_err(a, b))

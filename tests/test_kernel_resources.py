@@ -16,7 +16,7 @@ def _tile(algo, cells, storage="d", red=0):
 
 
 NOOP, CAYLEY, BLOCH = "9algo_noop", "11algo_cayleyILi%dEE", \
-    "13algo_bloch2_tILb0EE"
+    "13algo_bloch2_tILi0EE"
 
 
 @pytest.mark.parametrize("name,waves,scratch", [
