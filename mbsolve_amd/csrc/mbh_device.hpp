@@ -999,6 +999,15 @@ __device__ __forceinline__ void taylor_sincos(double x, double& s, double& c)
     c = fma(pc, x2, 1.0);
 }
 
+/* the same coefficients, sin then cos (1/13! .. -1/3!, -1/14! .. 1/4!) */
+static __constant__ const double TAYLOR_COEFF[12] = {
+    1.6059043836821614599e-10,  -2.5052108385441718775e-08,
+    2.7557319223985890653e-06,  -1.9841269841269841270e-04,
+    8.3333333333333333333e-03,  -1.6666666666666666667e-01,
+    -1.1470745597729724714e-11, 2.0876756987868098979e-09,
+    -2.7557319223985890653e-07, 2.4801587301587301587e-05,
+    -1.3888888888888888889e-03, 4.1666666666666666667e-02,
+};
 
 /* sin and cos of a small angle x, by wave-uniform tier of max |x|:
  * TIER 0: |x| <= 2^-13, x - x^3/6 and 1 - x^2/2 (relative truncation
@@ -1615,9 +1624,13 @@ struct algo_zform {
     {
         R.k.pin();
         double sn[B], cs[B], r[K];
-        /* wave-uniform tier, as in update_multi_p; the ranges beyond 2^-5 in
-         * a rolled loop (one copy of the library function; unrolled, its
-         * registers would halve the wavefronts per SIMD) */
+        /* wave-uniform tier, as in update_multi_p.  Up to 0.25 its series (on
+         * a field of 0.12 per step, 262144 cells of three levels, 1000 steps,
+         * 5.71 -> 3.37 ms against the library function); three levels take
+         * it from 2^-10 on, a tier less in the chain of tests (16384 cells,
+         * weak field, 4000 steps 3.13 -> 2.82 ms).  The library function in
+         * a rolled loop (one copy; unrolled, its registers would halve the
+         * wavefronts per SIMD). */
         const double xm = mine ? R.thmax * fabs(e) : 0.0;
         auto tier = [&](auto t) {
 #pragma unroll
@@ -1629,8 +1642,28 @@ struct algo_zform {
             tier(std::integral_constant<int, 0>());
         } else if (__all(xm <= 0x1p-10)) {
             tier(std::integral_constant<int, 1>());
-        } else if (__all(xm <= 0x1p-5)) {
+        } else if (N > 3 && __all(xm <= 0x1p-5)) {
             tier(std::integral_constant<int, 4>());
+        } else if (__all(xm <= TAYLOR_MAX)) {
+            /* (coefficients from memory, by an address that the compiler
+             * cannot see through: as literals they would be kept in
+             * registers over the steps) */
+            int off = 0;
+            asm volatile("" : "+s"(off));
+            cdp tc = (cdp)TAYLOR_COEFF + off;
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                const double x = R.th[b] * e, x2 = x * x;
+                double ps = tc[0], pc = tc[6];
+#pragma unroll
+                for (int i = 1; i < 6; i++) {
+                    ps = fma(ps, x2, tc[i]);
+                    pc = fma(pc, x2, tc[6 + i]);
+                }
+                pc = fma(pc, x2, -0.5);
+                sn[b] = fma(ps * x2, x, x);
+                cs[b] = fma(pc, x2, 1.0);
+            }
         } else {
             double ws[B], wc[B];
 #pragma unroll 1

@@ -850,3 +850,32 @@ def test_bloch_real_dipole_and_mixed_hamiltonian(gpu, form, tile):
                        capi.split_records(prob, out[0][0]), ref):
         assert np.max(np.abs(b)) > 0.0, r["type"]
         assert rel_err(a, b) <= tol, (r["type"], rel_err(a, b))
+
+
+@pytest.mark.parametrize("levels", [3, 4])
+@pytest.mark.parametrize("angle", [5e-4, 5e-3, 0.028, 0.12, 0.24, 0.6])
+def test_zform_one_cell_per_lane_angle_ranges(gpu, levels, angle):
+    """Three- and four-level z-form at one cell per lane, the largest plane
+    angle of the first step in each range of its sin and cos: the oracle's
+    populations on the trace-1 scale, fields relative to their maximum, to
+    1e-10 (the z-form's bound)."""
+    spec = setups.marskar2011(levels, num_gridpoints=160, endtime=0.02e-12)
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, "zform"), dev, scen)
+    blobs = np.array(prob["zform_consts"]).reshape(
+        int(prob["num_materials"]), -1)
+    B = (levels * levels - 1) // 2
+    spec["sources"] = []
+    spec["e_init"] = angle / max(np.max(np.abs(q[3:3 + B]))
+                                 for q in blobs if q[0] != 0.0)
+    spec["rho_init"] = ([1.0] + [0.0] * (levels - 1), [])
+    iv = spec["endtime"] / 6
+    spec["records"] = [{"name": n, "interval": iv} for n in ("inv12", "e")]
+    sol = _solve(spec, "zform", temporal_block=8, tile_cells=64)
+    ref = oracle.OracleRun(sol.problem()).run().records()
+    for r, b in zip(sol.get_results(), ref):
+        a = r.get_data_real()
+        assert np.max(np.abs(b)) > 0.0, r.get_name()
+        err = (float(np.max(np.abs(a - b))) if r.get_name()[0] == "i"
+               else rel_err(a, b))
+        assert err <= 1e-10, (r.get_name(), err)
