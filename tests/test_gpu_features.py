@@ -879,3 +879,133 @@ def test_zform_one_cell_per_lane_angle_ranges(gpu, levels, angle):
         err = (float(np.max(np.abs(a - b))) if r.get_name()[0] == "i"
                else rel_err(a, b))
         assert err <= 1e-10, (r.get_name(), err)
+
+
+@pytest.mark.parametrize("levels,form,order,tol", [
+    (3, "fp64", "plain", 1e-12), (5, "fp64", "plain", 1e-12),
+    (6, "fp64", "plain", 1e-12), (3, "fp64", "red", 1e-12),
+    (6, "fp64", "red", 1e-12), (3, "zform64", "plain", 1e-10),
+    (4, "zform64", "plain", 1e-10), (6, "zform64", "plain", 1e-10),
+    (4, "mfma64", "plain", 1e-6), (6, "mfma64", "plain", 1e-6)])
+def test_many_sources_and_records_rodrigues(gpu, levels, form, order, tol):
+    """Twelve sources and 27 point records of every kind, all due at every
+    step, within one tile of one medium: the sources beyond the register and
+    the staged ones, the records beyond the staged ones, with a cell's rows
+    over several wavefronts, by one, and on the matrix cores; against the
+    oracle (populations on the trace-1 scale, fields relative to their
+    maximum)."""
+    spec = setups.marskar2011(levels, num_gridpoints=300, endtime=0.02e-12)
+    spec["regions"] = [("Active region", "AR_Marsk", 0.0, 1e-4)]
+    spec["endtime"] = 0.1e-12
+    dx = 1e-4 / 299
+    src = spec["sources"][0]
+    spec["sources"] = [
+        dict(src, name="g%d" % i, hard=i in (3, 8), ampl=1e8 * (i + 1),
+             position=(100.5 + 2 * (i // 2 if i < 2 else i)) * dx,
+             tau=1.5e-14, phase=3e-14 + 2e-15 * i) for i in range(12)]
+    spec["records"] = [
+        {"name": "r%d" % i, "type": (0, 1, 2, 4)[i % 4], "row": 1, "col": 1,
+         "interval": 0.0, "position": (103 + i % 20) * dx}
+        for i in range(27 - levels)]
+    spec["records"] += [{"name": "d%d%d" % (i, i), "type": 3, "row": i,
+                         "col": i, "interval": 0.0, "position": 110 * dx}
+                        for i in range(1, levels + 1)]
+    suffix = {"fp64": "", "zform64": "zform"}.get(form, form)
+    dev, scen = setups.build(spec)
+    prob = mb.build_problem(setups.solver_name(spec, suffix, order), dev,
+                            scen)
+    print("case many rodr", levels, form, order, flush=True)
+    ctx = capi.Context([prob], capi.options(form, temporal_block=12,
+                                            tile_cells=64, order=order))
+    assert (ctx.info()["mfma_tiles"] > 0) == (form == "mfma64")
+    ctx.run(0, int(prob["num_timesteps"]))
+    got = capi.split_records(prob, ctx.records(0))
+    ctx.close()
+    # (two threads: the red oracle skips a source at the first halo cell of
+    # a thread's chunk, as the reference does)
+    ref = oracle.OracleRun(prob).run(order=order, threads=2).records()
+    for r, a, b in zip(prob["records"], got, ref):
+        assert np.max(np.abs(b)) > 0.0, r["type"]
+        err = (float(np.max(np.abs(a - b))) if r["type"] >= 3
+               else rel_err(a, b))
+        assert err <= tol, (r["type"], err)
+
+
+@pytest.mark.parametrize("levels,form", [(4, "mfma"), (4, "mfma64"),
+                                         (6, "mfma"), (6, "mfma64")])
+def test_matrix_core_runs_repeat_and_read_out(gpu, levels, form):
+    """Four and six levels on the matrix cores, uniform and mixed tiles: a
+    second run after mbh_reset gives the first one's records and state, and
+    the read-out without allocation gives the state, also in a batch."""
+    specs = []
+    for n in (700, 300):
+        spec = _planes_spec(levels)
+        spec["num_gridpoints"] = n
+        spec["sources"][0]["ampl"] = 5e8
+        specs.append(spec)
+    mb.material.clear_library()
+    probs = []
+    for spec in specs:
+        dev, scen = setups.build(spec, clear_library=False)
+        probs.append(mb.build_problem(setups.solver_name(spec, form), dev,
+                                      scen))
+    for batch in (probs[:1], probs[1:], [probs[1], probs[1]]):
+        print("case repeat", levels, form, flush=True)
+        ctx = capi.Context(batch, capi.options(form, temporal_block=8))
+        assert ctx.info()["mfma_tiles"] > 0
+        out = []
+        for _ in range(3):
+            ctx.run(0, int(batch[0]["num_timesteps"]))
+            out.append((ctx.records(0), ctx.state(0),
+                        ctx.state(0, noalloc=True)))
+            ctx.reset()
+        ctx.close()
+        rec, st, _ = out[0]
+        assert np.max(np.abs(rec)) > 0
+        for r2, s2, na in out:
+            assert np.array_equal(r2, rec)
+            for k in ("e", "h", "p", "d"):
+                assert np.array_equal(s2[k], st[k]), k
+                assert np.array_equal(na[k], st[k]), k
+
+
+@pytest.mark.parametrize("mfma,plain,tol", [("mfma64", "zform64", 1e-10),
+                                            ("mfma", "mixed", 1e-5)])
+@pytest.mark.parametrize("regions", [False, True])
+def test_three_level_mfma_forms_run_the_zform(gpu, mfma, plain, tol,
+                                              regions):
+    """Three levels: the MFMA forms issue no matrix instruction and give the
+    bits of the z-form with their state storage, within that form's bound of
+    the oracle."""
+    spec = setups.v3_rodr(num_gridpoints=1500, endtime=0.3e-12,
+                          num_records=8)
+    if regions:
+        name, mat, x0, x1 = spec["regions"][-1]
+        xs = [x0 + (x1 - x0) * f for f in (0.0, 0.3, 0.31, 1.0)]
+        spec["materials"]["gap"] = {}
+        spec["regions"][-1:] = [(name, mat, xs[0], xs[1]),
+                                ("gap", "gap", xs[1], xs[2]),
+                                (name + "2", mat, xs[2], xs[3])]
+    suffix = {"zform64": "zform"}
+    out = []
+    for form in (mfma, plain):
+        dev, scen = setups.build(spec)
+        prob = mb.build_problem(
+            setups.solver_name(spec, suffix.get(form, form)), dev, scen)
+        print("case three levels", form, regions, flush=True)
+        ctx = capi.Context([prob], capi.options(form, temporal_block=8,
+                                                tile_cells=64))
+        assert ctx.info()["mfma_tiles"] == 0
+        ctx.run(0, int(prob["num_timesteps"]))
+        out.append((ctx.records(0), ctx.state(0)))
+        ctx.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    for k in ("e", "h", "p", "d"):
+        assert np.array_equal(out[0][1][k], out[1][1][k]), k
+    ref = oracle.OracleRun(prob).run().records()
+    for r, a, b in zip(prob["records"],
+                       capi.split_records(prob, out[0][0]), ref):
+        assert np.max(np.abs(b)) > 0.0, r["type"]
+        err = (float(np.max(np.abs(a - b))) if r["type"] >= 3
+               else rel_err(a, b))
+        assert err <= tol, (r["type"], err)
