@@ -145,10 +145,12 @@ struct run_layout {
  * row-major) kept by the Bloch form: rho00, rho11, Re rho01, Im rho01. */
 constexpr uint32_t BLOCH_FROM_REF[4] = { 0, 6, 2, 3 };
 
-/* Bloch-form constants (layout in algo_bloch2) from the reference Cayley
- * blob of a two-level material (MBH_CAYLEY_STRIDE(2) doubles). */
+/* how far the trace factors may be from exactly 1 and 0 to be taken for
+ * rounding (bloch2_constants) */
 constexpr double TRACE_TOL = 2e-15;
 
+/* Bloch-form constants (layout in algo_bloch2) from the reference Cayley
+ * blob of a two-level material (MBH_CAYLEY_STRIDE(2) doubles). */
 void bloch2_constants(const double* cq, double* o)
 {
     typedef std::complex<double> cx;
@@ -1003,7 +1005,10 @@ void set_geometry(mbh_ctx* ctx, uint32_t C, uint32_t tb)
 }
 
 /* Per-tile source ranges (sources inside the loaded span, halo included)
- * and record lists (records overlapping the owned span). */
+ * and records (those overlapping the owned span).  Each tile has its own
+ * copies of its records' descriptors, 56 bytes each, which a launch then
+ * reads without an index in between: a tile owns at least eight cells, so
+ * a record's copies take less memory than one of its rows in the scratch. */
 int build_tile_tables(mbh_ctx* ctx, bool with_records)
 {
     const uint64_t nt = ctx->num_tiles;
@@ -1022,6 +1027,7 @@ int build_tile_tables(mbh_ctx* ctx, bool with_records)
         meta[t].src_lo = (uint32_t)(a - ctx->srcs.begin());
         meta[t].src_hi = (uint32_t)(b - ctx->srcs.begin());
     }
+    static_assert(sizeof(dev_record) == 56, "stated above");
     std::vector<dev_record> recs;
     if (with_records) {
         std::vector<std::pair<uint64_t, uint32_t>> tile_rec;
@@ -1176,12 +1182,6 @@ hipError_t launch_block(const mbh_ctx* ctx, KArgs k);
 constexpr uint32_t FP32_MIN_BLOCK = 8;
 constexpr double FP32_TIE = 0.015;
 
-/*
- * Autotuner: times every admissible (cells per lane, temporal block) pair
- * on the context's own state and picks the fastest per cell update.  The
- * trial launches read the current buffer, write the other one (discarded)
- * and record nothing, so the simulation state is untouched.
- */
 /* Largest number of tiles for the team form of the FP64 Rodrigues kernel.  It
  * does about the work of the one-wavefront kernel (a little more: E and H and
  * the LDS exchanges in every wavefront) with all SIMDs of a CU, so it wins
@@ -1211,6 +1211,12 @@ tile_launch_fn geometry_kernel(const mbh_ctx* ctx, uint32_t kform)
     return find_kernel(ctx->algo, ctx->levels, kform, ctx->C, ctx->order)->fn;
 }
 
+/*
+ * Autotuner: times every admissible (cells per lane, temporal block) pair
+ * on the context's own state and picks the fastest per cell update.  The
+ * trial launches read the current buffer, write the other one (discarded)
+ * and record nothing, so the simulation state is untouched.
+ */
 int autotune(mbh_ctx* ctx, uint32_t req_tb, uint32_t req_tile)
 {
     uint32_t kform = kernel_form(ctx->algo, ctx->levels, ctx->form);

@@ -246,7 +246,6 @@ struct algo_noop {
     struct state {
         double v[STATE];
     };
-    __device__ static bool has_qm(cdp) { return false; }
     __device__ static void update(cdp, state&, double, double&) {}
     template<int C>
     __device__ static void update_multi(cdp, state*, const double*, double*)
@@ -318,9 +317,8 @@ struct algo_cayley {
         }
     }
 
-    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
-    /* branch-free body; callers check has_qm */
+    /* branch-free body; only for media with a density */
     __device__ static void update(cdp q, state& s, double e, double& p)
     {
         ccp H0 = (ccp)(q + OFF_H0);
@@ -621,7 +619,6 @@ struct algo_bloch2_t {
         double v[STATE];
     };
 
-    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
     /* Constants of one material, loaded before the steps of a launch: from
      * a wave-uniform address they stay in SGPRs (read inside the step they
@@ -670,7 +667,8 @@ struct algo_bloch2_t {
     }
 
     /* 2 / n2 for n2 near 1: hardware reciprocal and one cubic step (with
-     * t = 1 - n2 r of at most 2^-20, r (1 + t + t^2) is off by t^3 / 2) */
+     * t = 1 - n2 r of at most 2^-20, r (1 + t + t^2) is off by a relative
+     * t^3) */
     __device__ static double two_over(double n2)
     {
         const double r = __builtin_amdgcn_rcp(n2);
@@ -831,9 +829,8 @@ struct algo_rodr {
     static constexpr int OFF_C1 = OFF_TH + B;
     static constexpr int OFF_C2 = OFF_C1 + B * K * K;
 
-    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
-    /* callers check has_qm */
+    /* only for media with a density */
     __device__ static void update(cdp q, state& s, double e, double& p)
     {
         const double M_CP = q[1];
@@ -1063,11 +1060,13 @@ __device__ __forceinline__ void tier_sincos(double x, double& s, double& c)
  * stay exact (a run that starts from noise has p = 0 until its coherences
  * grow, as in the reference form).  State: d, as algo_rodr.
  * Bound by the latency of one step's chain on grids that leave the SIMDs
- * one wavefront or none.  Whole runs, algo_rodr -> algo_rodrp: six-level
- * ladder, 8192 cells x 800 steps, 1702 -> 18.6 ms (algo_rodr: 93 kflop and
- * 10 KB of scratch per lane and step); five-level comb, 8192 x 600,
- * 239 -> 5.3 ms; three levels, 16384 x 8000, 112 -> 16.7 ms, and one cell,
- * 10000 steps, 102 -> 34 ms.
+ * one wavefront or none; with one wavefront per tile, whole runs, algo_rodr
+ * -> algo_rodrp: six-level ladder, 8192 cells x 800 steps, 1702 -> 18.6 ms
+ * (algo_rodr: 93 kflop and 10 KB of scratch per lane and step); five-level
+ * comb, 8192 x 600, 239 -> 5.3 ms; three levels, 16384 x 8000, 112 -> 16.7
+ * ms (11.2 from row registers); one cell, 10000 steps, 102 -> 34 ms.  Few
+ * tiles, and six levels in the plain order always, take team_kernel with the
+ * same arithmetic.
  *
  * Blob (STRIDE doubles): [0] has_qm  [1] number of planes  [2] pb
  *   [3] max theta dt   then c (K), pv (K), A1 (K^2),
@@ -1148,7 +1147,6 @@ struct algo_rodrp {
 
     static constexpr int STAGE = 0;
 
-    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
     /* o = A1 d + c: every row accumulates in ascending order; RG rows side
      * by side hide the FMA latency (more would spill at K = 35) */
@@ -1446,7 +1444,6 @@ struct algo_zform {
     static constexpr int DEV_STRIDE = OFF_POP + N * (K + 1);
     static constexpr bool SHIFT = true;
 
-    __device__ static bool has_qm(cdp q) { return q[0] != 0.0; }
 
     /* Small blobs (K <= 8) are staged in LDS by the tile kernel: W, c, a
      * and theta are then read from there every step instead of through

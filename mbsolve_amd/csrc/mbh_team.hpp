@@ -34,7 +34,7 @@ namespace mbh {
  * with 2, 4 .. 8 wavefronts: K = 8 1.52, -, 1.17, 8: 1.2; K = 15 5.24, 4:
  * 3.25, 5: 3.34, 8: 3.16 (and 5.1 instead of 3.4 with two tiles per CU);
  * K = 24 8.8, 4: 4.40, 6: 4.33, 8: 4.33; K = 35 24.4, 4: 7.75, 7: 8.2, 8: 8.4
- * (four hold 126 registers of constants each and use one SIMD each). */
+ * (four hold 128 registers of constants each and use one SIMD each). */
 template<int N>
 constexpr int team_waves()
 {

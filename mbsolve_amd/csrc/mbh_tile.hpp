@@ -440,9 +440,9 @@ constexpr int MAX_BLOCK = 64;   /* largest temporal block */
 /* Source values of a tile for the steps of the block: the first one's in a
  * register, one step per lane (REG: read by readlane; an LDS read in the
  * step's chain cost 165 of 410 cycles of the two-level Bloch step), the first
- * TILE_SOURCES otherwise in LDS, any more from memory.  where: offset of the source's
- * cell in the tile (the tile's first cell, halo included, has offset 0) and,
- * in bit 0, its type. */
+ * TILE_SOURCES otherwise in LDS, any more from memory.  where: offset of the
+ * source's cell in the tile (the tile's first cell, halo included, has offset
+ * 0) and, in bit 0, its type. */
 __device__ __forceinline__ uint32_t source_where(const KArgs& k, uint32_t i,
                                                  int64_t tile0)
 {
