@@ -187,7 +187,7 @@ __global__ __launch_bounds__(64 * team_waves<N>()) void team_kernel(KArgs k)
         d[i] = in ? d[i] : 0.0;
     }
     const dev_record rec_own = own_record(k, M, lane);
-    const tile_sources srcs = stage_sources<true>(k, lds.src, lane, wv == 0,
+    const tile_sources srcs = stage_sources<true>(k, lds, lane, wv == 0,
                                                   M, tile0, n0, nsteps);
     const double* f = k.fdtd + (uint64_t)(m < 0 ? 0 : m) * FDTD_STRIDE;
     const double fa = f[0], fb = f[1], fg = f[3], fx = f[4];
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(64 * team_waves<N>()) void team_kernel(KArgs k)
         const double h_right = from_right(h);
         double en = (m >= 0) ? fa * e + fb * (-fg * p + (h_right - h) * fx)
                              : 0.0;
-        for_sources<true>(k, lds.src, srcs, tile0, n0, s,
+        for_sources<true>(k, lds, srcs, tile0, n0, s,
                           [&](int32_t at, bool hard, double v)
                               __attribute__((always_inline)) {
                               const double x = hard ? v : en + v;

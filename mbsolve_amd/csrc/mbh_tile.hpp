@@ -434,15 +434,27 @@ __device__ __forceinline__ void add_shift(const KArgs& k, int32_t m,
     }
 }
 
-constexpr uint32_t TILE_SOURCES = 8; /* of a tile, staged in LDS */
+constexpr uint32_t TILE_SOURCES = 7; /* of a tile, staged in LDS */
 constexpr int MAX_BLOCK = 64;   /* largest temporal block */
+
+/* LDS of a tile: the sources' values for the block's steps and their places,
+ * the records */
+struct tile_lds {
+    double src[TILE_SOURCES][MAX_BLOCK];
+    rec_stage rec;
+    uint32_t where[TILE_SOURCES];
+};
+static_assert(sizeof(tile_lds) <= 4 * 1280, "see TILE_SOURCES");
 
 /* Source values of a tile for the steps of the block: the first one's in a
  * register, one step per lane (REG: read by readlane; an LDS read in the
- * step's chain cost 165 of 410 cycles of the two-level Bloch step), the first
- * TILE_SOURCES otherwise in LDS, any more from memory.  where: offset of the
- * source's cell in the tile (the tile's first cell, halo included, has offset
- * 0) and, in bit 0, its type. */
+ * step's chain cost 165 of 410 cycles of the two-level Bloch step), the next
+ * TILE_SOURCES in LDS, any more from memory.  Seven, so that tile_lds takes
+ * four of the LDS's units of 1280 bytes: in five, a CU holds 25 instead of 32
+ * tiles of the kernels that need 64 registers or fewer (noop, 2^26 cells, one
+ * cell per lane: FP64 8.4 -> 7.6 ms, FP32 6.6 -> 6.0 ms per 96 steps).
+ * where: offset of the source's cell in the tile (the tile's first cell, halo
+ * included, has offset 0) and, in bit 0, its type. */
 __device__ __forceinline__ uint32_t source_where(const KArgs& k, uint32_t i,
                                                  int64_t tile0)
 {
@@ -462,8 +474,8 @@ __device__ __forceinline__ double source_load(const KArgs& k, uint32_t i,
 }
 template<bool REG>
 __device__ __forceinline__ tile_sources stage_sources(
-    const KArgs& k, double (*S)[MAX_BLOCK], int lane, bool writer,
-    const tile_meta& M, int64_t tile0, uint64_t n0, uint32_t nsteps)
+    const KArgs& k, tile_lds& S, int lane, bool writer, const tile_meta& M,
+    int64_t tile0, uint64_t n0, uint32_t nsteps)
 {
     tile_sources T{ M.src_lo, M.src_hi - M.src_lo, 0u, 0.0 };
     if (T.count > 0) {
@@ -473,12 +485,17 @@ __device__ __forceinline__ tile_sources stage_sources(
             T.where0 = source_where(k, T.lo, tile0);
             T.v0 = source_load(k, T.lo, n, in);
         }
-        if (T.count > (REG ? 1u : 0u)) {
+        constexpr uint32_t J0 = REG ? 1u : 0u;
+        if (T.count > J0) {
             if (writer) {
-                const uint32_t cnt =
-                    T.count < TILE_SOURCES ? T.count : TILE_SOURCES;
-                for (uint32_t j = REG ? 1u : 0u; j < cnt; j++) {
-                    S[j][lane] = source_load(k, T.lo + j, n, in);
+                const uint32_t cnt = T.count - J0 < TILE_SOURCES
+                    ? T.count - J0
+                    : TILE_SOURCES;
+                for (uint32_t j = 0; j < cnt; j++) {
+                    S.src[j][lane] = source_load(k, T.lo + J0 + j, n, in);
+                    if (lane == 0) {
+                        S.where[j] = source_where(k, T.lo + J0 + j, tile0);
+                    }
                 }
             }
             __syncthreads();
@@ -490,7 +507,7 @@ __device__ __forceinline__ tile_sources stage_sources(
  * order (solver_cpu_fdtd.tpp:247-255) */
 template<bool REG, typename F>
 __device__ __forceinline__ void for_sources(const KArgs& k,
-                                            const double (*S)[MAX_BLOCK],
+                                            const tile_lds& S,
                                             const tile_sources& T,
                                             int64_t tile0, uint64_t n0,
                                             uint32_t s, F&& put)
@@ -502,23 +519,24 @@ __device__ __forceinline__ void for_sources(const KArgs& k,
         put((int32_t)(T.where0 >> 1), (T.where0 & 1u) != 0u,
             lane_f64(T.v0, (int)s));
     }
-    for (uint32_t j = REG ? 1u : 0u; j < T.count; j++) {
-        const uint32_t w = source_where(k, T.lo + j, tile0);
+    /* (rolled: unrolled over the staged ones, their places would be read
+     * ahead of the steps into scalar registers) */
+    constexpr uint32_t J0 = REG ? 1u : 0u;
+#pragma unroll 1
+    for (uint32_t j = J0; j < T.count; j++) {
+        uint32_t w;
         double v;
-        if (j < TILE_SOURCES) {
-            v = S[j][s];
+        if (j < J0 + TILE_SOURCES) {
+            w = S.where[j - J0];
+            v = S.src[j - J0][s];
         } else {
+            w = source_where(k, T.lo + j, tile0);
             v = as_const(k.src_data)[(uint64_t)(T.lo + j) * k.n_t + n0 + s];
         }
         put((int32_t)(w >> 1), (w & 1u) != 0u, v);
     }
 }
 
-/* LDS of a tile: the sources' values for the block's steps, the records */
-struct tile_lds {
-    double src[TILE_SOURCES][MAX_BLOCK];
-    rec_stage rec;
-};
 
 /* One tile t: all steps of the temporal block for the tile's cells.
  * With W > 1 the tile spans W wavefronts of one workgroup, each holding a
@@ -553,22 +571,30 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
                        as_const(k.tiles)[t].rec_lo,
                        as_const(k.tiles)[t].rec_hi };
 
-    /* The tile's records: staged before the state is loaded they cost
-     * registers of their own only; one cell per lane with its constants in
-     * registers (grids bound by the latency of a launch), and the two-level
-     * Cayley form without its zeros (2^20 cells, 9.1 us per step against
-     * 9.3), have the descriptors in flight together with the state.  Staged after the constants, and
-     * with the record code's addresses kept over the steps, the FP64 noop
-     * kernel spilled (2^27 cells, tiles of 512 cells, blocks of 32 steps:
-     * 65 -> 72 us per step) and three-level Cayley fitted one wavefront per
-     * SIMD instead of two (2^18 cells 14.8 -> 17.4 us per step, 14.5 here). */
-    constexpr bool STAGE_LATE = (C == 1 && (A::CONSTS || A::ROWC)) ||
-        std::is_same<A, algo_cayley2r>::value;
+    /* When the tile's records are staged.  Before the state is loaded they
+     * cost registers of their own only.  One cell per lane with constants in
+     * registers (grids bound by the latency of a launch) has the descriptors
+     * in flight together with the state and stages them after the constants
+     * (two-level Bloch form, 8192 cells x 16000 steps: 3.73 ms, 3.90 with
+     * the constants loaded after it); two-level Cayley without its zeros
+     * stages them between the two (2^20 cells, 9.1 us per step, 9.3 before
+     * the state).  Staged after the constants by every kernel, and with the
+     * record code's addresses kept over the steps, the FP64 noop kernel
+     * spilled (2^27 cells, tiles of 512 cells, blocks of 32 steps: 65 -> 72
+     * us per step) and three-level Cayley fitted one wavefront per SIMD
+     * instead of two (2^18 cells 14.8 -> 17.4 us per step, 14.3 here). */
+    constexpr bool STAGE_LAST = C == 1 && (A::CONSTS || A::ROWC);
+    constexpr bool STAGE_FIRST =
+        !STAGE_LAST && !std::is_same<A, algo_cayley2r>::value;
     uint64_t rec_steps = 0; /* steps of this block with a due record */
-    if constexpr (!STAGE_LATE) {
-        rec_steps =
-            stage_records(k, lds.rec, own_record(k, M, lane), lane, wv == 0,
-                          M, own_lo, own_hi, n0, nsteps);
+    auto stage = [&](const dev_record& R) __attribute__((always_inline)) {
+        if (M.rec_lo != M.rec_hi) {
+            rec_steps = stage_records(k, lds.rec, R, lane, wv == 0, M, own_lo,
+                                      own_hi, n0, nsteps);
+        }
+    };
+    if constexpr (STAGE_FIRST) {
+        stage(own_record(k, M, lane));
     }
 
     double e[C], h[C], p[C];
@@ -614,10 +640,12 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
             d[c].v[j] = in ? dv[j] : 0.0;
         }
     }
-    if constexpr (STAGE_LATE) {
-        rec_steps =
-            stage_records(k, lds.rec, own_record(k, M, lane), lane, wv == 0,
-                          M, own_lo, own_hi, n0, nsteps);
+    dev_record rec_own{};
+    if constexpr (!STAGE_FIRST) {
+        rec_own = own_record(k, M, lane);
+    }
+    if constexpr (!STAGE_FIRST && !STAGE_LAST) {
+        stage(rec_own);
     }
     /* the tile's sources, the first in a register; the larger z-forms and
      * four or more cells per lane with a density (but for the two-level
@@ -625,7 +653,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
     constexpr bool SRC_REG = A::DC < 24 &&
         (C < 4 || A::DC == 0 || bloch_real<A>);
     const tile_sources srcs =
-        stage_sources<SRC_REG>(k, lds.src, lane, wv == 0, M, tile0, n0,
+        stage_sources<SRC_REG>(k, lds, lane, wv == 0, M, tile0, n0,
                                nsteps);
 #pragma unroll
     for (int c = 0; c < C; c++) {
@@ -699,6 +727,10 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
             x_h[wv] = h[0];
         }
         __syncthreads();
+    }
+
+    if constexpr (STAGE_LAST) {
+        stage(rec_own);
     }
 
     /* material constants held over the steps: each lane's own with one cell
@@ -853,7 +885,7 @@ __device__ __forceinline__ void tile_body(const KArgs& k, uint64_t t,
         }
 
         /* sources, in list order (solver_cpu_fdtd.tpp:247-255) */
-        for_sources<SRC_REG>(k, lds.src, srcs, tile0, n0, s,
+        for_sources<SRC_REG>(k, lds, srcs, tile0, n0, s,
                     [&](int32_t at, bool hard, double v)
                         __attribute__((always_inline)) {
                         const int32_t off =

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
 
     /* sources and records of this tile */
     const tile_sources srcs =
-        stage_sources<(N < 5)>(k, lds.src, lane, true, M, g0, n0, nsteps);
+        stage_sources<(N < 5)>(k, lds, lane, true, M, g0, n0, nsteps);
     const uint64_t rec_steps = stage_records(
         k, lds.rec, rec_own, lane, true, M, own_lo, own_hi, n0, nsteps);
 
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(64) ZM_OCCUPANCY void zm_kernel(KArgs k)
         const double h_right = from_right(h);
         double en = fma(fx, h_right - h, fma(fg, p, fa * e));
         /* sources, in list order */
-        for_sources<(N < 5)>(k, lds.src, srcs, g0, n0, s,
+        for_sources<(N < 5)>(k, lds, srcs, g0, n0, s,
                     [&](int32_t at, bool hard, double v)
                         __attribute__((always_inline)) {
                         if (at == lane) {

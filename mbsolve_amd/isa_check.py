@@ -178,8 +178,10 @@ def check(path):
 
 
 def resources(path):
-    """{mangled kernel name: {"vgpr", "agpr", "vgpr_spills", "scratch"}}"""
+    """{mangled kernel name: {"vgpr", "agpr", "sgpr", "lds", "vgpr_spills",
+    "scratch"}}"""
     keys = {".agpr_count": "agpr", ".vgpr_count": "vgpr",
+            ".sgpr_count": "sgpr", ".group_segment_fixed_size": "lds",
             ".vgpr_spill_count": "vgpr_spills",
             ".private_segment_fixed_size": "scratch"}
     out = {}

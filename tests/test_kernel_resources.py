@@ -1,5 +1,7 @@
 """Registers and scratch of the built kernels whose speed on large grids hangs
-on the wavefronts that fit a SIMD (512 vector registers, in units of eight)."""
+on the wavefronts that fit a SIMD: 512 vector registers in units of eight, 800
+scalar registers in units of sixteen, 160 KB of LDS per four SIMDs in units of
+1280 bytes."""
 import pytest
 
 from mbsolve_amd import capi, isa_check
@@ -20,6 +22,10 @@ NOOP, CAYLEY, BLOCH = "9algo_noop", "11algo_cayleyILi%dEE", \
 
 
 @pytest.mark.parametrize("name,waves,scratch", [
+    (_tile(NOOP, 1), 8, 0), (_tile(NOOP, 1, red=1), 8, 0),
+    (_tile("14algo_noop_fast", 1, "f"), 8, 0), (_tile("13algo_noop_hz0", 1, "f"),
+                                            8, 0),
+    (_tile("13algo_noop_hz0", 2, "f"), 8, 0),
     (_tile(NOOP, 2), 8, 0), (_tile(NOOP, 4), 5, 0), (_tile(NOOP, 8), 3, 0),
     (_tile(NOOP, 4, red=1), 5, 0),
     (_tile(CAYLEY % 2, 1), 4, 0), (_tile(CAYLEY % 2, 4), 2, 48),
@@ -30,4 +36,7 @@ NOOP, CAYLEY, BLOCH = "9algo_noop", "11algo_cayleyILi%dEE", \
 def test_wavefronts_fit(kernels, name, waves, scratch):
     k = kernels[name]
     assert 512 // (-(-k["vgpr"] // 8) * 8) >= waves, k
+    assert 800 // (-(-k["sgpr"] // 16) * 16) >= waves, k
+    # one wavefront per workgroup
+    assert 163840 // (-(-k["lds"] // 1280) * 1280) >= 4 * waves, k
     assert k["scratch"] <= scratch, k
